@@ -74,7 +74,7 @@ static int tape_fluid(fsibe_sim *s, bool explicit_step) {
   const int j = t.n;
   adj_copy_d(s->stream, reinterpret_cast<const double *>(s->T[0]), reinterpret_cast<double *>(t.A + j * t.NH),
              2 * t.NH);
-  adj_copy_d(s->stream, reinterpret_cast<const double *>(s->T[1]), reinterpret_cast<double *>(t.B + j * t.NH),
+  adj_copy_d(s->stream, reinterpret_cast<const double *>(s->Bp), reinterpret_cast<double *>(t.B + j * t.NH),
              2 * t.NH);
   adj_copy_d(s->stream, s->u1, t.u1 + j * t.N, t.N);
   adj_copy_d(s->stream, s->u2, t.u2 + j * t.N, t.N);
@@ -520,7 +520,7 @@ static int adj_record_reverse(fsibe_adjoint *a, int k, double *J, double *T, dou
   // pipelined as fsibe_run's prescribed-motion loop: the host prepares
   // step j+1 while step j runs and reads each step's results one step late
   for (int j = 0; j < len && rc == FSIBE_OK; ++j) {
-    rc = run_one(s, true, false);
+    rc = run_one(s, true, false, j + 1 < len);
     if (rc == FSIBE_OK) {
       t.rec[j].dt1 = s->dt1;
       if (t.n != j + 1) rc = set_err(FSIBE_ESTATE, "adjoint: step %d was not recorded", first + j);
@@ -531,6 +531,8 @@ static int adj_record_reverse(fsibe_adjoint *a, int k, double *J, double *T, dou
   }
   s->tape = nullptr;
   s->pipe = false;
+  s->k1_ready = false;
+  s->k2_ready = false;
   if (s->res_pending) {  // the last step's results (the reverse sweep needs none of them)
     if (hipStreamSynchronize(s->stream) != hipSuccess && rc == FSIBE_OK) rc = set_err(FSIBE_EHIP, "adjoint: sync failed");
     parse_results(s, s->slot ^ 1);

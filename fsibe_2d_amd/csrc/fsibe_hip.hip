@@ -31,6 +31,7 @@
 #include "kernels.hpp"
 #include "kernels_mask.hpp"
 #include "kernels_step.hpp"
+#include "kernels_fused.hpp"
 #include "kernels_adjoint.hpp"
 #include "kinematics.hpp"
 #include "solid.hpp"
@@ -354,6 +355,67 @@ static int pick_tx(int H, int ny, int nfld, int split) {
 static bool size_ok(int nx, int ny) {
   FftPlan a, b;
   return nx >= 4 && ny >= 4 && nx % 2 == 0 && ny % 2 == 0 && make_plan(nx / 2, a) && make_plan(ny, b);
+}
+
+// fn(shape) for the fused column stage (K4, K5 and the dw/dy column) of
+// columns of length ny; false if the grid has none (the separate stages run).
+// The shapes follow from what a workgroup holds: four slots of one column up
+// to 512 points, of two columns (32-byte row pieces) at 768 and 1024, two
+// slots of two columns at 1536, and one buffer of two columns beyond, where
+// the fields follow one another.  Both sides measured on square grids (one
+// simulation, K4 + K5 with four fields + the dw/dy column of K1, us):
+// 256^2 19.0 -> 7.2, 384^2 22.9 -> 11.3, 512^2 21.3 -> 11.7, 768^2 30.7 ->
+// 22.1, 1024^2 37.9 -> 26.0, 2048^2 131 -> 125.
+template <class Fn>
+static bool with_col_step(int ny, int H, bool px, Fn &&fn) {
+  (void)px;
+  switch (ny) {
+    case 64: fn(ColStepShape<64, 1, 8, 4, false>{}); return true;
+    case 96: fn(ColStepShape<96, 1, 12, 4, false>{}); return true;
+    case 128: fn(ColStepShape<128, 1, 16, 4, false>{}); return true;
+    case 192: fn(ColStepShape<192, 1, 24, 4, false>{}); return true;
+    case 256: fn(ColStepShape<256, 1, 32, 4, false>{}); return true;
+    case 384: fn(ColStepShape<384, 1, 48, 4, false>{}); return true;
+    case 512: fn(ColStepShape<512, 1, 64, 4, false>{}); return true;
+    default: break;
+  }
+  if (H % 2) return false;
+  switch (ny) {
+    case 768: fn(ColStepShape<768, 2, 96, 4, true>{}); return true;
+    case 1024: fn(ColStepShape<1024, 2, 128, 4, true>{}); return true;
+    case 1536: fn(ColStepShape<1536, 2, 192, 2, true>{}); return true;
+    case 2048:
+      if (px) fn(ColStepShape<2048, 2, 256, 0, true>{});
+      else fn(ColStepShape<2048, 2, 256, 0, false>{});
+      return true;
+    case 4096:
+      if (px) return false;
+      fn(ColStepShape<4096, 2, 512, 0, false>{});
+      return true;
+    default: return false;
+  }
+}
+
+// fn(shape) for the fused row stage (K6 and the convective part of the next
+// K2) of rows of H complex values on ny rows; false if there is none
+template <class Fn>
+static bool with_row_step(int H, int ny, Fn &&fn) {
+  switch (H) {
+    case 32:
+      if (ny % 4) return false;
+      fn(RowStepShape<32, 4, 4, 4, false>{});
+      return true;
+    case 64:
+      if (ny % 2) return false;
+      fn(RowStepShape<64, 8, 4, 2, false>{});
+      return true;
+    case 96: fn(RowStepShape<96, 16, 4, 1, false>{}); return true;
+    case 128: fn(RowStepShape<128, 16, 4, 1, false>{}); return true;
+    case 192: fn(RowStepShape<192, 32, 4, 1, false>{}); return true;
+    case 256: fn(RowStepShape<256, 32, 4, 1, false>{}); return true;
+    case 512: fn(RowStepShape<512, 64, 4, 1, true>{}); return true;
+    default: return false;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -939,7 +1001,8 @@ struct fsibe_sim {
   // by every wait that follows the copies)
   int upload_pending = 0;
   double2 *twx, *twy;
-  double2 *W[2], *NL[2], *T[7];
+  char *fields = nullptr;  // the allocation that holds the fields of the grid below
+  double2 *W[2], *NL[2], *T[9];
   double *u1, *u2, *vor_mean, *ms, *wallrow;
   double *frame = nullptr;   // iSponge = 22: the frame mask (SmoothFrameAroundDomain), full grid
   double *rowpen = nullptr;  // iMeanVelocity = 11: row sums of the penalisation term (2 per row)
@@ -979,10 +1042,14 @@ struct fsibe_sim {
   hipEvent_t ev_dt;
   hipEvent_t ev_step;        // after a step's last kernel (iFLUSI=1 loop)
   // the next step's first column pass (it reads only vortk) already runs:
-  // launched for time level k1_level before the host solves the beam
+  // launched for time level k1_level before the host solves the beam, or
+  // part of the previous step's fused column stage.  Its dw/dy column is in
+  // Bp (T[1] or T[7]), its omega column in T[0]
   bool k1_ready = false;
-  // K2's convective part of every row launched ahead with K1 (iFLUSI=1 loop)
+  // K2's convective part of every row went ahead too (the iFLUSI=1 loop's
+  // launch, or the previous step's fused row stage), into Rcp (T[2] or T[8])
   bool k2_ready = false;
+  double2 *Bp = nullptr, *Rcp = nullptr;
   // launch choices of the column stages K1, K4, K5, K7 (the autotuner's,
   // once fsibe_run has measured them for this grid; else the static ones)
   ColSel csel[4];
@@ -1372,10 +1439,8 @@ extern "C" int fsibe_sim_destroy(fsibe_sim *s) {
   if (!s) return FSIBE_OK;
   open_gate(s);
   (void)hipStreamSynchronize(s->stream);
-  void *ptrs[] = {s->twx, s->twy, s->W[0], s->W[1], s->NL[0], s->NL[1], s->T[0], s->T[1], s->T[2], s->T[3],
-                  s->T[4], s->T[5], s->T[6], s->u1, s->u2, s->vor_mean, s->ms, s->wallrow,
-                  s->umax_part, s->dscal, s->mask_m, s->mask_vx, s->mask_vy, s->fb_p, s->fb_sa,
-                  s->fb_sb, s->d_stage, s->frame, s->rowpen, s->snap};
+  void *ptrs[] = {s->twx, s->twy, s->fields, s->ms, s->wallrow, s->umax_part, s->dscal, s->d_stage, s->frame,
+                  s->rowpen, s->snap};
   if (s->spec) fsibe_spectral_destroy(s->spec);
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
@@ -1474,22 +1539,22 @@ extern "C" int fsibe_sim_create(const fsibe_params *pp, fsibe_sim **out) {
   SIMCHK(hipMalloc(&s->twy, sizeof(double2) * s->ny));
   SIMCHK(hipMemcpy(s->twx, tx.data(), sizeof(double2) * s->nx, hipMemcpyHostToDevice));
   SIMCHK(hipMemcpy(s->twy, ty.data(), sizeof(double2) * s->ny, hipMemcpyHostToDevice));
-  for (int i = 0; i < 2; ++i) {
-    SIMCHK(hipMalloc(&s->W[i], sizeof(double2) * NH));
-    SIMCHK(hipMalloc(&s->NL[i], sizeof(double2) * NH));
-    SIMCHK(hipMemset(s->W[i], 0, sizeof(double2) * NH));
-    SIMCHK(hipMemset(s->NL[i], 0, sizeof(double2) * NH));
+  {
+    // every field of the grid in one allocation (22 of them: each call of
+    // the allocator costs more than the fields' clearing), the ones that
+    // are read before they are written cleared
+    const size_t fld = (sizeof(double2) * NH + 255) & ~(size_t)255;
+    SIMCHK(hipMalloc(&s->fields, 22 * fld));
+    SIMCHK(hipMemset(s->fields, 0, 14 * fld));
+    char *q = s->fields;
+    auto take = [&](auto &dst) { dst = reinterpret_cast<std::remove_reference_t<decltype(dst)>>(q); q += fld; };
+    for (int i = 0; i < 2; ++i) { take(s->W[i]); take(s->NL[i]); }
+    for (int i = 0; i < 7; ++i) take(s->T[i]);
+    take(s->u1); take(s->u2); take(s->vor_mean);
+    take(s->T[7]); take(s->T[8]);
+    take(s->mask_m); take(s->mask_vx); take(s->mask_vy);
+    take(s->fb_p); take(s->fb_sa); take(s->fb_sb);
   }
-  for (int i = 0; i < 7; ++i) {
-    SIMCHK(hipMalloc(&s->T[i], sizeof(double2) * NH));
-    SIMCHK(hipMemset(s->T[i], 0, sizeof(double2) * NH));
-  }
-  SIMCHK(hipMalloc(&s->u1, sizeof(double) * N));
-  SIMCHK(hipMalloc(&s->u2, sizeof(double) * N));
-  SIMCHK(hipMalloc(&s->vor_mean, sizeof(double) * N));
-  SIMCHK(hipMemset(s->u1, 0, sizeof(double) * N));
-  SIMCHK(hipMemset(s->u2, 0, sizeof(double) * N));
-  SIMCHK(hipMemset(s->vor_mean, 0, sizeof(double) * N));
   SIMCHK(hipMalloc(&s->umax_part, sizeof(double) * s->ny));
   SIMCHK(hipMemset(s->umax_part, 0, sizeof(double) * s->ny));
   SIMCHK(hipMalloc(&s->dscal, sizeof(DevScalars)));
@@ -1503,12 +1568,6 @@ extern "C" int fsibe_sim_create(const fsibe_params *pp, fsibe_sim **out) {
   SIMCHK(hipHostMalloc((void **)&s->h_res, 2 * s->res_stride, hipHostMallocMapped | hipHostMallocCoherent));
   memset(s->h_res, 0, 2 * s->res_stride);
   SIMCHK(hipHostGetDevicePointer((void **)&s->d_res, s->h_res, 0));
-  SIMCHK(hipMalloc(&s->mask_m, sizeof(double) * N));
-  SIMCHK(hipMalloc(&s->mask_vx, sizeof(double) * N));
-  SIMCHK(hipMalloc(&s->mask_vy, sizeof(double) * N));
-  SIMCHK(hipMalloc(&s->fb_p, sizeof(double) * N));
-  SIMCHK(hipMalloc(&s->fb_sa, sizeof(double) * N));
-  SIMCHK(hipMalloc(&s->fb_sb, sizeof(double) * N));
   const int nsb = std::max(s->nb * s->ns, 1);
   // staging layout
   {
@@ -2105,14 +2164,17 @@ static int velocity_only(fsibe_sim *s, double time) {
 
 // K1: A = Fy^-1[W0], B = Fy^-1[i ky W0] (and Fy^-1[i ky psi] for iSponge =
 // 10, whose outflow sponge acts inside the penalisation term).  It reads only
-// the vorticity of time level `level`.
-static int launch_k1(fsibe_sim *s, int level) {
+// the vorticity of time level `level`.  have_a: T[0] holds that level's
+// omega column already (the column stage just before wrote it).
+static int launch_k1(fsibe_sim *s, int level, bool have_a = false) {
   const bool sp10 = s->p.iSponge == 10 && s->penal_on && s->ms;
   double2 *outs[3] = {s->T[0], s->T[1], s->T[4]};
   const int fsel[3] = {0, 4, 2};
+  const int f0 = have_a && !sp10 ? 1 : 0;
   PROF_BEGIN(s, P_COLS_W0);
-  CHK(cols_inv_fields(s, s->W[level], outs, fsel, sp10 ? 3 : 2));
+  CHK(cols_inv_fields(s, s->W[level], outs + f0, fsel + f0, (sp10 ? 3 : 2) - f0));
   prof_end(s, P_COLS_W0);
+  s->Bp = s->T[1];
   return FSIBE_OK;
 }
 
@@ -2130,20 +2192,49 @@ static int launch_k2_ahead(fsibe_sim *s) {
   none.m = none.vx = none.vy = nullptr;
   const size_t lds = sizeof(double2) * 3 * padlen(s->H);
   CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
-    KLAUNCH(k_rows_nl<decltype(F)>, na + nb, nt, lds, s->stream, s->T[0], s->T[1], s->u1, s->u2,
+    KLAUNCH(k_rows_nl<decltype(F)>, na + nb, nt, lds, s->stream, s->T[0], s->Bp, s->u1, s->u2,
             s->sponge_on ? s->ms : nullptr, none, (int)s->penal_on, s->T[2], s->penal_on ? s->T[3] : nullptr,
             F, s->twx, s->sc,
             s->umax_part, s->ny, s->dscal, s->fp, 0.0, 0.0, 0, res_dev(s, s->slot), 0, na, b1 + 1, 0,
             s->penal_on ? s->rowpen : nullptr, (int)(s->p.iSponge == 10));
     return FSIBE_OK;
   }));
+  s->Rcp = s->T[2];
   s->k2_ready = true;
   return FSIBE_OK;
 }
 
+static RowStepArgs row_step_args(const fsibe_sim *s, const MaskBox &mb) {
+  RowStepArgs a;
+  a.Cw = s->T[0]; a.Cpsi = s->T[1]; a.Cpsiy = s->T[2]; a.Cwy = s->T[7];
+  a.u1 = s->u1; a.u2 = s->u2; a.vor_mean = s->vor_mean; a.ms = s->sponge_on ? s->ms : nullptr;
+  a.mb = mb; a.win = s->win[0]; a.win2 = s->win[1];
+  a.sums = rows_dev(s, s->slot); a.umax_part = s->umax_part;
+  a.Rq = s->T[4]; a.Rqy = s->T[5]; a.Rc = s->T[8];
+  a.s = s->dscal; a.c = s->sc;
+  return a;
+}
+static ColStepArgs col_step_args(const fsibe_sim *s, const MaskBox &mb, const double2 *Rc, bool explicit_step,
+                                 bool next) {
+  ColStepArgs a;
+  // without penalisation K2 leaves Rpx unwritten (it is 0) and the stage skips it
+  a.Rc = Rc; a.Rpx = s->penal_on ? s->T[3] : nullptr;
+  a.W0 = s->W[s->n0]; a.NL1 = s->NL[s->n1]; a.NL0 = s->NL[s->n0]; a.W1 = s->W[s->n1];
+  a.o[0] = s->T[0]; a.o[1] = s->T[1]; a.o[2] = s->T[2];
+  a.o[3] = s->forces_on && s->visc ? s->T[3] : nullptr;
+  a.o[4] = next ? s->T[7] : nullptr;
+  a.s = s->dscal; a.explicit_step = explicit_step;
+  rpx_rows(s, mb, a.py0, a.py1);
+  stress_rows(s, a.r0, a.r1);
+  a.c = s->sc;
+  return a;
+}
+
 // K1 .. K6 of a step: the new vorticity, velocity, pressure right-hand
-// sides and the row sums
-static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_step) {
+// sides and the row sums.  next: another step follows in the same call, and
+// its dw/dy column and convective term are formed here, where their inputs
+// are at hand
+static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_step, bool next = false) {
   if (s->p.iBeam > 0 && !s->have_beam) return set_err(FSIBE_ESTATE, "fsibe_create_mask must be called first");
   std::vector<double>().swap(s->restored);
   if (!s->have_beam)  // no beam: walls / cylinder only (create_mask.f90:34-69)
@@ -2164,6 +2255,7 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
     CHK(launch_k1(s, n0));
   }
   MaskBox mb = mask_box(s);
+  if (!k2_ahead) s->Rcp = s->T[2];
   // K2 (block 0 also computes the K3 scalars from the previous u_max partials).
   // When the convective part of every row went ahead, the penalisation of
   // this mask box's rows remains.
@@ -2173,17 +2265,21 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
     if (k2_ahead) {
       const int y0 = mb.x1 >= mb.x0 ? mb.y0 : 0, nrow = mb.x1 >= mb.x0 ? mb.y1 - mb.y0 + 1 : 0;
       CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
-        KLAUNCH(k_rows_pen<decltype(F)>, nrow + 1, nt, lds, s->stream, s->u1, s->u2, mb, s->T[2], s->T[3],
-                F, s->twx, s->sc, y0, nrow, s->rowpen, s->umax_part, s->ny, s->dscal, s->fp, time, dt0,
-                (int)explicit_step, res_dev(s, s->slot));
+        if (s->pipe)
+          KLAUNCH_EV(k_rows_pen<decltype(F)>, nrow + 1, nt, lds, s->stream, s->ev_dt, s->u1, s->u2, mb, s->Rcp, s->T[3],
+                     F, s->twx, s->sc, y0, nrow, s->rowpen, s->umax_part, s->ny, s->dscal, s->fp, time, dt0,
+                     (int)explicit_step, res_dev(s, s->slot));
+        else
+          KLAUNCH(k_rows_pen<decltype(F)>, nrow + 1, nt, lds, s->stream, s->u1, s->u2, mb, s->Rcp, s->T[3],
+                  F, s->twx, s->sc, y0, nrow, s->rowpen, s->umax_part, s->ny, s->dscal, s->fp, time, dt0,
+                  (int)explicit_step, res_dev(s, s->slot));
         return FSIBE_OK;
       }));
-      if (s->pipe) HIPCHK(hipEventRecord(s->ev_dt, s->stream));
     } else if (s->pipe) {
       // ev_dt at K2's end: the host reads dt1 and then the previous step's
       // results (kernels before this one in the stream)
       CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
-        KLAUNCH_EV(k_rows_nl<decltype(F)>, s->ny, nt, lds, s->stream, s->ev_dt, s->T[0], s->T[1], s->u1, s->u2,
+        KLAUNCH_EV(k_rows_nl<decltype(F)>, s->ny, nt, lds, s->stream, s->ev_dt, s->T[0], s->Bp, s->u1, s->u2,
                    s->sponge_on ? s->ms : nullptr, mb, (int)s->penal_on, s->T[2], s->penal_on ? s->T[3] : nullptr,
                    F, s->twx, s->sc,
                    s->umax_part, s->ny, s->dscal, s->fp, time, dt0, (int)explicit_step, res_dev(s, s->slot), 0,
@@ -2192,7 +2288,7 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
       }));
     } else {
       CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
-        KLAUNCH(k_rows_nl<decltype(F)>, s->ny, nt, lds, s->stream, s->T[0], s->T[1], s->u1, s->u2,
+        KLAUNCH(k_rows_nl<decltype(F)>, s->ny, nt, lds, s->stream, s->T[0], s->Bp, s->u1, s->u2,
                 s->sponge_on ? s->ms : nullptr, mb, (int)s->penal_on, s->T[2], s->penal_on ? s->T[3] : nullptr,
                 F, s->twx, s->sc,
                 s->umax_part, s->ny, s->dscal, s->fp, time, dt0, (int)explicit_step, res_dev(s, s->slot), 0, s->ny,
@@ -2222,23 +2318,34 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
       }));
     }
   }
-  // K4
-  {
-    PROF_BEGIN(s, P_COLS_AB2);
+  // K4, K5: the fused column stage where the grid has one
+  next = next && !sp10 && s->p.iMeanVelocity != 11;
+  int rc = FSIBE_OK;
+  PROF_BEGIN(s, P_COLS_AB2);
+  const bool fused_cols = with_col_step(s->ny, s->H, s->penal_on, [&](auto S) {
+    using ST = decltype(S);
+    rc = [&]() -> int {
+      KLAUNCH(k_col_step<ST>, s->H / ST::TX, ST::THREADS, ST::LDS, s->stream,
+              col_step_args(s, mb, s->Rcp, explicit_step, next), s->twy);
+      return FSIBE_OK;
+    }();
+  });
+  CHK(rc);
+  if (!fused_cols) {
     CHK(with_cols_sel<2>(s->py, s->H, sim_sel(s, 1, 1), [&](auto F, int nt, int TX) -> int {
       const size_t lds = k4_lds(s->ny, s->penal_on, TX);
       int py0, py1;
       rpx_rows(s, mb, py0, py1);
       // without penalisation K2 leaves Rpx unwritten (it is 0) and K4 skips it
-      KLAUNCH(k_cols_ab2<decltype(F)>, s->H / TX, nt, lds, s->stream, s->T[2], s->penal_on ? s->T[3] : nullptr,
+      KLAUNCH(k_cols_ab2<decltype(F)>, s->H / TX, nt, lds, s->stream, s->Rcp, s->penal_on ? s->T[3] : nullptr,
               s->W[n0], s->NL[n1],
               s->NL[n0], s->W[n1], s->dscal, (int)explicit_step, F, s->twy, s->sc, py0, py1);
       return FSIBE_OK;
     }));
-    prof_end(s, P_COLS_AB2);
   }
-  // K5: omega, psi, i ky psi (, -ky^2 psi) of vortk(n1)
-  {
+  prof_end(s, P_COLS_AB2);
+  if (!fused_cols) {
+    // K5: omega, psi, i ky psi (, -ky^2 psi) of vortk(n1)
     const bool st = s->forces_on && s->visc;
     double2 *outs[4] = {s->T[0], s->T[1], s->T[2], s->T[3]};
     const int fsel[4] = {0, 1, 2, 3};
@@ -2248,20 +2355,43 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
     CHK(cols_inv_fields(s, s->W[n1], outs, fsel, st ? 4 : 3, 2, r0_3, r1_3));
     prof_end(s, P_COLS_W1);
   }
-  // K6
+  // K6, with the next step's convective term where the grid has the fused
+  // row stage and the column stage left it the dw/dy column
+  bool conv = false;
   {
     const size_t lds = sizeof(double2) * 3 * padlen(s->H);
     PROF_BEGIN(s, P_ROWS_PRESS);
-    CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
-      // the step's instances: mode 1, with or without the pressure rhs
-      using FT = decltype(F);
-      auto *kern = s->pressure_on ? &k_rows_press<FT, 1, 1> : &k_rows_press<FT, 1, 0>;
-      KLAUNCH(kern, s->ny, nt, lds, s->stream, s->T[0], s->T[1], s->T[2], s->u1, s->u2, s->vor_mean, mb, s->win[0],
-              s->win[1], rows_dev(s, s->slot), s->umax_part, s->T[4], s->T[5], s->dscal, 0.0, 0.0, 1,
-              (int)s->pressure_on, F, s->twx, s->sc);
-      return FSIBE_OK;
-    }));
+    const bool fused_rows = with_row_step(s->H, s->ny, [&](auto S) {
+      using ST = decltype(S);
+      conv = next && fused_cols;
+      auto *kern = s->pressure_on ? (conv ? &k_row_step<ST, true, true> : &k_row_step<ST, true, false>)
+                                  : (conv ? &k_row_step<ST, false, true> : &k_row_step<ST, false, false>);
+      rc = [&]() -> int {
+        KLAUNCH(kern, s->ny / ST::RPB, ST::THREADS, ST::LDS, s->stream, row_step_args(s, mb), s->twx);
+        return FSIBE_OK;
+      }();
+    });
+    CHK(rc);
+    if (!fused_rows)
+      CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
+        // the step's instances: mode 1, with or without the pressure rhs
+        using FT = decltype(F);
+        auto *kern = s->pressure_on ? &k_rows_press<FT, 1, 1> : &k_rows_press<FT, 1, 0>;
+        KLAUNCH(kern, s->ny, nt, lds, s->stream, s->T[0], s->T[1], s->T[2], s->u1, s->u2, s->vor_mean, mb, s->win[0],
+                s->win[1], rows_dev(s, s->slot), s->umax_part, s->T[4], s->T[5], s->dscal, 0.0, 0.0, 1,
+                (int)s->pressure_on, F, s->twx, s->sc);
+        return FSIBE_OK;
+      }));
     prof_end(s, P_ROWS_PRESS);
+  }
+  if (next && fused_cols) {
+    s->k1_ready = true;
+    s->k1_level = n1;
+    s->Bp = s->T[7];
+    if (conv) {
+      s->k2_ready = true;
+      s->Rcp = s->T[8];
+    }
   }
   s->slot_fluid[s->slot] = true;  // the host adds the row sums of K6
   return FSIBE_OK;
@@ -2298,8 +2428,8 @@ static int evolve_pressure_box(fsibe_sim *s) {
   return FSIBE_OK;
 }
 
-static int evolve(fsibe_sim *s, double time, double dt0, bool explicit_step) {
-  CHK(evolve_fluid(s, time, dt0, explicit_step));
+static int evolve(fsibe_sim *s, double time, double dt0, bool explicit_step, bool next = false) {
+  CHK(evolve_fluid(s, time, dt0, explicit_step, next));
   return evolve_pressure_box(s);
 }
 
@@ -2606,8 +2736,8 @@ static void integrate_all(fsibe_sim *s, double time) {
 // One step of the loop.  pipe: do not wait for the step to finish; wait only
 // for dt1 (written by the nonlinear-term kernel), read the previous step's
 // results, and return so that the host prepares the next step's geometry
-// while this one runs.
-static int run_one(fsibe_sim *s, bool pipe, bool k1_ahead) {
+// while this one runs.  next (pipe): another step follows in this call.
+static int run_one(fsibe_sim *s, bool pipe, bool k1_ahead, bool next = false) {
   s->pipe = pipe;
   const fsibe_params &p = s->p;
   const bool moving = (p.iSponge >= 4 && s->time < p.T_fullspeed) || p.iFLUSI == 1 || p.iMotion > 0;
@@ -2633,7 +2763,7 @@ static int run_one(fsibe_sim *s, bool pipe, bool k1_ahead) {
     CHK(evolve_fluid(s, s->time, s->startup_done ? s->dt0 : 0.0, !s->startup_done));
     CHK(evolve_pressure_box(s));
   } else {
-    CHK(evolve(s, s->time, s->startup_done ? s->dt0 : 0.0, !s->startup_done));
+    CHK(evolve(s, s->time, s->startup_done ? s->dt0 : 0.0, !s->startup_done, pipe && next));
   }
   // iFLUSI=1 with the next step ahead: ev_step at the force kernel's end,
   // carried by its dispatch (a marker after it would idle the queue first)
@@ -2642,7 +2772,7 @@ static int run_one(fsibe_sim *s, bool pipe, bool k1_ahead) {
   if (!pipe && k1_ahead) {
     // iFLUSI=1: the next step's K1 runs while the host solves the beam
     if (!step_recorded) HIPCHK(hipEventRecord(s->ev_step, s->stream));
-    CHK(launch_k1(s, s->n1));
+    CHK(launch_k1(s, s->n1, true));
     s->k1_ready = true;
     s->k1_level = s->n1;
     CHK(launch_k2_ahead(s));
@@ -2729,7 +2859,7 @@ extern "C" int fsibe_run(fsibe_sim *s, int nsteps, fsibe_step_out *out) {
     // the next step's first kernel goes ahead of the host's beam solve when
     // there is a next step in this call (event timing keeps the plain order)
     const bool ahead = fsi && !s->prof.on && k + 1 < nsteps;
-    rc = run_one(s, pipe, ahead);
+    rc = run_one(s, pipe, ahead, k + 1 < nsteps);
     if (rc != FSIBE_OK) break;
     if (s->last.status == 1) break;  // continue_timestep = .false.
   }
@@ -2967,7 +3097,8 @@ class HostPool {
 enum BatchStage { B_MASK, B_K1, B_K2, B_K4, B_K5, B_K6, B_K7, B_K8, B_K10, B_NST };
 
 static const size_t kBatchArgSize[B_NST] = {sizeof(MaskArgs),      sizeof(ColsInvArgs),   sizeof(RowsNlArgs),
-                                            sizeof(ColsAb2Args),   sizeof(ColsInvArgs),   sizeof(RowsPressArgs),
+                                            sizeof(ColsAb2Args),   sizeof(ColsInvArgs),
+                                            std::max(sizeof(RowsPressArgs), sizeof(RowStepRec)),
                                             sizeof(ColsPressArgs), sizeof(RowsBoxArgs),   sizeof(ForcesArgs)};
 
 struct BatchGroup {
@@ -3405,7 +3536,15 @@ static void fill_batch_args(fsibe_batch *b, BatchGroup &g, int j, fsibe_sim *s, 
     stress_rows(s, a.r0_3, a.r1_3);
     maxblk[B_K5] = std::max(maxblk[B_K5], a.nblk);
   }
-  {  // K6
+  // K6: the record of the row stage the single path launches
+  const bool rs = with_row_step(s->H, s->ny, [&](auto S) {
+    RowStepRec &r = reinterpret_cast<RowStepRec *>(A + g.off[B_K6])[j];
+    r.a = row_step_args(s, mb);
+    r.nblk = s->ny / decltype(S)::RPB;
+    r.pad = 0;
+    maxblk[B_K6] = std::max(maxblk[B_K6], r.nblk);
+  });
+  if (!rs) {
     RowsPressArgs &a = reinterpret_cast<RowsPressArgs *>(A + g.off[B_K6])[j];
     a.Cw = s->T[0]; a.Cpsi = s->T[1]; a.Cpsiy = s->T[2]; a.u1 = s->u1; a.u2 = s->u2; a.vor_mean = s->vor_mean;
     a.sums = rows_dev(s, s->slot); a.umax_part = s->umax_part; a.mb = mb; a.win = s->win[0];
@@ -3503,13 +3642,26 @@ static int batch_stages(fsibe_batch *b, const std::vector<std::array<int, B_NST>
             return FSIBE_OK;
           }));
           break;
-        case B_K6:
+        case B_K6: {
+          int rc = FSIBE_OK;
+          const bool rs = with_row_step(s0->H, s0->ny, [&](auto S) {
+            using ST = decltype(S);
+            auto *kern = g.pres ? &kb_row_step<ST, true, false> : &kb_row_step<ST, false, false>;
+            rc = [&]() -> int {
+              SLAUNCH(kern, gx, nm, ST::THREADS, ST::LDS, g.stream, mode,
+                      reinterpret_cast<const RowStepRec *>(arr(g, B_K6)), s0->twx);
+              return FSIBE_OK;
+            }();
+          });
+          CHK(rc);
+          if (rs) break;
           CHK(with_rows<3>(s0->px, [&](auto F, int nt) -> int {
             SLAUNCH(kb_rows_press<decltype(F)>, gx, nm, nt, sizeof(double2) * 3 * padlen(s0->H), g.stream, mode,
                     reinterpret_cast<const RowsPressArgs *>(arr(g, B_K6)), F, s0->twx);
             return FSIBE_OK;
           }));
           break;
+        }
         case B_K7:
           CHK(with_cols_sel<2>(s0->py, s0->H, g.sel[B_K7], [&](auto F, int nt, int TX) -> int {
             SLAUNCH(kb_cols_press<decltype(F)>, gx, nm, nt, sizeof(double2) * 2 * TX * padlen(s0->ny), g.stream, mode,

@@ -1,0 +1,53 @@
+"""The fused column and row stages of the time loop (kernels_fused.hpp): a run
+of several steps in one call forms each next step's dw/dy column and
+convective term inside the stages of the step before, a run of one step per
+call forms them with kernels of their own.  Both do the same operations on
+every value, so the fields and the loads agree bit for bit: no tolerance."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# every shape of the two stages, and lengths that have one of them or none
+GRIDS = [(64, 64), (128, 96), (96, 128), (192, 192), (256, 64), (64, 256), (384, 384), (512, 192), (1024, 768),
+         (256, 1024), (384, 1536), (72, 96), (128, 2048), (1024, 1024)]
+
+
+def _run(p, steps, split):
+    from fsibe_2d_amd.inputs import half_to_packed, normals
+    from fsibe_2d_amd.solver import FluidSim
+
+    z = np.zeros((p.ny, p.nx // 2), dtype=np.complex128)
+    g = normals(5, 2 * 6 * 7).reshape(2, 6, 7)
+    z[1:7, :7] = 1e-3 * (g[0] + 1j * g[1])
+    z[1:7, 0] = 0.0  # kx = 0 needs its conjugate row
+    s = FluidSim(p)
+    s.set_vortk(half_to_packed(z))
+    if split:
+        for _ in range(steps):
+            out = s.run(1)
+    else:
+        out = s.run(steps)
+    got = [s.field(f) for f in ("vortk", "nlk", "u1", "u2", "vor_mean")]
+    b = s.beam()
+    s.close()
+    return got, out, b
+
+
+@pytest.mark.parametrize("nx,ny", GRIDS)
+@pytest.mark.parametrize("kind", ["beam", "loads off", "no body"])
+def test_one_call_of_several_steps_equals_several_calls_of_one(nx, ny, kind):
+    from fsibe_2d_amd import Params
+
+    p = Params(nx=nx, ny=ny, ns=33, nu=2e-3, dt_fixed=2e-4)
+    if kind == "loads off":
+        p = p.replace(iSaveBeam=0, iSponge=0)
+    if kind == "no body":
+        p = p.replace(iBeam=0, iSaveBeam=0, iSponge=0, iMotion=0, iMeanVelocity=4)
+    a, oa, ba = _run(p, 4, False)
+    b, ob, bb = _run(p, 4, True)
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
+    for k in ("dt1", "u_max", "Force", "Force_press", "energies", "bsi"):
+        assert oa[k] == ob[k], k
+    assert np.array_equal(ba["pressure"], bb["pressure"]) and np.array_equal(ba["tau"], bb["tau"])
