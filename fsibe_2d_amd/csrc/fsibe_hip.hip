@@ -396,6 +396,14 @@ static bool with_col_step(int ny, int H, bool px, Fn &&fn) {
   }
 }
 
+// transform lengths that a policy fixes at compile time (0: a runtime plan),
+// so that the fallbacks below are not instantiated where they cannot run
+template <class F> struct fixed_len { static constexpr int v = 0; };
+template <int H, int NT> struct fixed_len<RowCT<H, NT>> { static constexpr int v = H; };
+template <int NY, int TX, int NT> struct fixed_len<ColCT<NY, TX, NT>> { static constexpr int v = NY; };
+constexpr bool always_col_step(int ny) { return ny == 128 || ny == 256 || ny == 384 || ny == 512; }
+constexpr bool always_row_step(int H) { return H == 128 || H == 192 || H == 256 || H == 512; }
+
 // fn(shape) for the fused row stage (K6 and the convective part of the next
 // K2) of rows of H complex values on ny rows; false if there is none
 template <class Fn>
@@ -2101,7 +2109,7 @@ static int create_mask_impl(fsibe_sim *s, double time, const double *x, const do
     dim3 blk(kMaskThreads);
     dim3 grd(std::max(tiles_x, bg.fwg), tiles_y + (bg.fwg > 0 ? 1 : 0));
     PROF_BEGIN(s, P_MASK);
-    k_mask<<<grd, blk, sizeof(int4) * std::max(s->nprim, 1), s->stream>>>(
+    k_mask<<<grd, blk, 0, s->stream>>>(
         reinterpret_cast<const Prim *>(s->d_stage + s->off_prim), s->nprim, s->wallrow ? s->wallrow + 0 : nullptr, mc,
         bg, tiles_y, s->mbox.x0, s->mbox.y0, s->mbox.w(), s->mbox.h(), s->mask_m, s->mask_vx, s->mask_vy,
         s->mask_win);
@@ -2337,9 +2345,10 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
       int py0, py1;
       rpx_rows(s, mb, py0, py1);
       // without penalisation K2 leaves Rpx unwritten (it is 0) and K4 skips it
-      KLAUNCH(k_cols_ab2<decltype(F)>, s->H / TX, nt, lds, s->stream, s->Rcp, s->penal_on ? s->T[3] : nullptr,
-              s->W[n0], s->NL[n1],
-              s->NL[n0], s->W[n1], s->dscal, (int)explicit_step, F, s->twy, s->sc, py0, py1);
+      if constexpr (!always_col_step(fixed_len<decltype(F)>::v))
+        KLAUNCH(k_cols_ab2<decltype(F)>, s->H / TX, nt, lds, s->stream, s->Rcp, s->penal_on ? s->T[3] : nullptr,
+                s->W[n0], s->NL[n1],
+                s->NL[n0], s->W[n1], s->dscal, (int)explicit_step, F, s->twy, s->sc, py0, py1);
       return FSIBE_OK;
     }));
   }
@@ -2376,10 +2385,12 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
       CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
         // the step's instances: mode 1, with or without the pressure rhs
         using FT = decltype(F);
-        auto *kern = s->pressure_on ? &k_rows_press<FT, 1, 1> : &k_rows_press<FT, 1, 0>;
-        KLAUNCH(kern, s->ny, nt, lds, s->stream, s->T[0], s->T[1], s->T[2], s->u1, s->u2, s->vor_mean, mb, s->win[0],
-                s->win[1], rows_dev(s, s->slot), s->umax_part, s->T[4], s->T[5], s->dscal, 0.0, 0.0, 1,
-                (int)s->pressure_on, F, s->twx, s->sc);
+        if constexpr (!always_row_step(fixed_len<FT>::v)) {
+          auto *kern = s->pressure_on ? &k_rows_press<FT, 1, 1> : &k_rows_press<FT, 1, 0>;
+          KLAUNCH(kern, s->ny, nt, lds, s->stream, s->T[0], s->T[1], s->T[2], s->u1, s->u2, s->vor_mean, mb, s->win[0],
+                  s->win[1], rows_dev(s, s->slot), s->umax_part, s->T[4], s->T[5], s->dscal, 0.0, 0.0, 1,
+                  (int)s->pressure_on, F, s->twx, s->sc);
+        }
         return FSIBE_OK;
       }));
     prof_end(s, P_ROWS_PRESS);
@@ -3116,7 +3127,6 @@ struct BatchGroup {
   float tune_us[B_NST], base_us[B_NST];  // measured time of the choice and of the static one (0: not tuned)
   int ncand[B_NST];   // choices measured
   int cap[B_NST];     // grid.x of the stage in the captured step (0: stage left out)
-  int nprim_cap = 1;  // the members' largest room for mask primitives (the mask stage's LDS)
   // the group's stages as two captured graphs (up to the nonlinear term, and
   // the rest), replayed on the group's stream
   hipGraph_t graph[2] = {nullptr, nullptr};
@@ -3423,7 +3433,6 @@ extern "C" int fsibe_batch_create(const fsibe_params *params, int n, const doubl
     }
     g->px = g->px || s->penal_on;
     g->mem.push_back(i);
-    g->nprim_cap = std::max(g->nprim_cap, s->nprim_cap);
   }
   size_t off = 0;
   for (auto &g : b->groups)
@@ -3617,7 +3626,7 @@ static int batch_stages(fsibe_batch *b, const std::vector<std::array<int, B_NST>
       if (gx <= 0) continue;
       switch (k) {
         case B_MASK:
-          SLAUNCH(kb_mask, gx, nm, kMaskThreadsBatch, sizeof(int4) * g.nprim_cap, g.stream, mode,
+          SLAUNCH(kb_mask, gx, nm, kMaskThreadsBatch, 0, g.stream, mode,
                   reinterpret_cast<const MaskArgs *>(arr(g, B_MASK)));
           break;
         case B_K1:
@@ -3656,8 +3665,9 @@ static int batch_stages(fsibe_batch *b, const std::vector<std::array<int, B_NST>
           CHK(rc);
           if (rs) break;
           CHK(with_rows<3>(s0->px, [&](auto F, int nt) -> int {
-            SLAUNCH(kb_rows_press<decltype(F)>, gx, nm, nt, sizeof(double2) * 3 * padlen(s0->H), g.stream, mode,
-                    reinterpret_cast<const RowsPressArgs *>(arr(g, B_K6)), F, s0->twx);
+            if constexpr (!always_row_step(fixed_len<decltype(F)>::v))
+              SLAUNCH(kb_rows_press<decltype(F)>, gx, nm, nt, sizeof(double2) * 3 * padlen(s0->H), g.stream, mode,
+                      reinterpret_cast<const RowsPressArgs *>(arr(g, B_K6)), F, s0->twx);
             return FSIBE_OK;
           }));
           break;

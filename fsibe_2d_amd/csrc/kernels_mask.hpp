@@ -55,16 +55,27 @@ __device__ __forceinline__ double angle_deg(double g, double pi) {
   return a * 180.0 / pi;
 }
 
-// One workgroup of four waves per 8x8 tile of the mask box (lane = pixel).
-// The bounding boxes of all primitives are first copied to LDS.  Then, in
-// passes over the primitive list, the ones whose boxes meet the tile are
-// compacted in drawing order (ballot) and staged in LDS; the four waves
-// evaluate the staged primitives' profile values at the tile's pixels in
-// parallel (the erf / sqrt / atan2 work, which does not depend on the running
-// maximum), and wave 0 applies them in drawing order with the reference's
-// replacement rule.  A value of -1 marks "primitive does not touch this
-// pixel" (every profile value is >= 0 and so is the running maximum); the
-// sharp end marks "not touched" with -2 and otherwise overwrites.
+// One workgroup per 8x8 tile of the mask box (lane = pixel).  In passes over
+// the primitive list, the ones whose boxes meet the tile are compacted in
+// drawing order (a ballot per wave, a prefix over the waves) and staged in
+// LDS; each wave tests a run of them against the tile's 64 pixels and leaves
+// the distance where one covers a pixel; the covered (primitive, pixel) pairs
+// are compacted in turn, and all threads evaluate the profile (two erf) on
+// those alone; then each wave reduces its run and wave 0 joins the runs, with
+// the reference's replacement rule: a later primitive replaces the value only
+// where it is larger (strict >), which is the maximum with the first index
+// winning ties, so runs may be joined in any grouping.  The sharp end
+// overwrites instead: a pass that holds it is applied in sequence by wave 0.
+// A value of -1 marks "primitive does not touch this pixel" (every profile
+// value is >= 0 and so is the running maximum); the sharp end marks "not
+// touched" with -2.
+//
+// The kernel is a latency chain (launch, two dependent loads, barriers) on a
+// few hundred workgroups; a straight stretch of beam covers a pixel with one
+// or two of the ~30 primitives that meet its tile, so evaluating the profile
+// on covered pairs only takes out most of the arithmetic, and a list searched
+// by all waves at once most of the chain: 12.5 -> 8.6 us at 1024^2 (a tile
+// grid of 37 x 5, ~170 primitives), 14.3 -> 9.4 us at 256^2.
 constexpr int kMaskTile = 8;
 constexpr int kMaskPix = kMaskTile * kMaskTile;  // pixels per tile = lanes of a wave
 // waves per tile: 8 for one simulation's mask (its ~200 tiles leave most
@@ -75,8 +86,10 @@ constexpr int kMaskThreads = kMaskPix * kMaskWaves, kMaskThreadsBatch = kMaskPix
 constexpr int kMaxTilePrims = 1024;  // >= number of primitives (host checks)
 constexpr int kMaskStage = 64;       // primitives staged per pass (one pass for a tile of the beam)
 
-// profile value of primitive P at (xi, yj), or -1 / -2 (see above)
-__device__ __forceinline__ double prim_value(const Prim &P, const MaskConsts &c, int i, int j, double xi,
+// distance argument of primitive P's profile at (xi, yj) where it covers that
+// pixel, else -1; for the sharp end, whose profile is a product of two steps,
+// the value itself, or -2 (see above)
+__device__ __forceinline__ double prim_reach(const Prim &P, const MaskConsts &c, int i, int j, double xi,
                                              double yj) {
 #pragma clang fp contract(off)
   const double none = P.type == PRIM_SHARP ? -2.0 : -1.0;
@@ -87,7 +100,7 @@ __device__ __forceinline__ double prim_value(const Prim &P, const MaskConsts &c,
     const double xs = xi * a[4] - yj * a[5];
     const double ys = xi * a[5] + yj * a[4];
     if (xs >= a[0] && xs <= a[2] && ys <= (a[1] + a[6]) && ys >= (a[3] - a[6]))
-      return smooth_step(c, fabs(ys - a[1]), c.t, c.h);
+      return fabs(ys - a[1]);
     return -1.0;
   }
   if (P.type == PRIM_HINGE) {
@@ -118,13 +131,12 @@ __device__ __forceinline__ double prim_value(const Prim &P, const MaskConsts &c,
     } else if (b2 >= 270.0) {
       in2 = (gamma >= 90.0 + b2 - 360.0 && gamma < 270.0 + b2 - 360.0);
     }
-    return (in1 && in2) ? smooth_step(c, R, c.t, c.h) : -1.0;
+    return (in1 && in2) ? R : -1.0;
   }
   if (P.type == PRIM_DOT) {
     // DrawADot :690-701; a = px py vx vy t
     const double ddx = xi - a[0], ddy = yj - a[1];
-    const double R = sqrt(ddx * ddx + ddy * ddy);
-    return smooth_step(c, R, a[4], c.h);
+    return sqrt(ddx * ddx + ddy * ddy);
   }
   // PRIM_SHARP, DrawSharpEnd :825-847; a = p1s(2) p2s(2) cos sin t_star vx vy mdx
   const double xs = xi * a[4] + yj * a[5];
@@ -208,21 +220,17 @@ __device__ __forceinline__ void mask_body(const Prim *__restrict__ prims, int np
                                           double *__restrict__ om, double *__restrict__ ovx,
                                           double *__restrict__ ovy, int *__restrict__ owin, int tbx, int tby) {
 #pragma clang fp contract(off)
-  extern __shared__ int4 bnd[];  // ix0, ix1, iy0, iy1 of the np primitives (dynamic LDS, np entries)
   __shared__ Prim sp[kMaskStage];
   __shared__ int list[kMaskStage];
   __shared__ double val[kMaskStage][kMaskPix];
-  __shared__ int nstage, pnext;
+  __shared__ unsigned short pair[kMaskStage * kMaskPix];
+  __shared__ double rv[WAVES][kMaskPix];  // a wave's run: largest value, its staged index
+  __shared__ int ri[WAVES][kMaskPix];
+  __shared__ int cnt[WAVES], npair, sharp_in;
   const int tid = threadIdx.x, lane = tid & (kMaskPix - 1), wv = tid / kMaskPix;
   const int tx0 = bx0 + tbx * kMaskTile, ty0 = by0 + tby * kMaskTile;
   const int tx1 = tx0 + kMaskTile - 1, ty1 = ty0 + kMaskTile - 1;
   constexpr int NTHR = kMaskPix * WAVES;
-  for (int p = tid; p < np; p += NTHR) {
-    const int4 h = reinterpret_cast<const int4 *>(prims + p)[0];  // type ix0 ix1 iy0
-    bnd[p] = make_int4(h.y, h.z, h.w, prims[p].iy1);
-  }
-  if (tid == 0) pnext = 0;
-  __syncthreads();
   const int lx = tbx * kMaskTile + (lane & (kMaskTile - 1));
   const int ly = tby * kMaskTile + (lane / kMaskTile);
   const bool valid = lx < bw && ly < bh;
@@ -230,83 +238,115 @@ __device__ __forceinline__ void mask_body(const Prim *__restrict__ prims, int np
   const double xi = (double)i * c.dx, yj = (double)j * c.dy;
   double m = (valid && wallrow) ? wallrow[j] : 0.0, mvx = 0.0, mvy = 0.0;
   int wi = -1;
-  while (true) {
-    // wave 0 compacts the next primitives that meet the tile, in order
-    if (wv == 0) {
-      int p0 = pnext, n = 0;
-      while (p0 < np) {
-        const int p = p0 + lane;
-        bool f = false;
-        if (p < np) {
-          const int4 b = bnd[p];
-          f = !(b.y < tx0 || b.x > tx1 || b.w < ty0 || b.z > ty1);
+  // winner wi of this pass (staged index q): the velocity it sets
+  auto velocity = [&](int q) {
+    const Prim &P = sp[q];
+    const double *a = P.a;
+    if (P.type == PRIM_SEG) {
+      const double xs = xi * a[4] - yj * a[5];
+      mvx = (a[7] + (xs - a[0]) * (a[9] - a[7]) / c.ds);
+      mvy = (a[8] + (xs - a[0]) * (a[10] - a[8]) / c.ds);
+    } else if (P.type == PRIM_HINGE) {
+      mvx = a[5]; mvy = a[6];
+    } else {
+      mvx = a[2]; mvy = a[3];
+    }
+  };
+  // groups of NTHR primitives, each taken in rounds of kMaskStage of those
+  // that meet the tile
+  for (int p0 = 0; p0 < np; p0 += NTHR) {
+    const int p = p0 + tid;
+    bool f = false;
+    int type = 0;
+    if (p < np) {
+      const int4 h = reinterpret_cast<const int4 *>(prims + p)[0];  // type ix0 ix1 iy0
+      const int iy1 = prims[p].iy1;
+      type = h.x;
+      f = !(h.z < tx0 || h.y > tx1 || iy1 < ty0 || h.w > ty1);
+    }
+    const unsigned long long bal = __ballot(f);
+    if (lane == 0) cnt[wv] = __popcll(bal);
+    __syncthreads();
+    int pos = __popcll(bal & ((1ull << lane) - 1ull)), tot = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      if (w < wv) pos += cnt[w];
+      tot += cnt[w];
+    }
+    for (int r0 = 0; r0 < tot; r0 += kMaskStage) {
+      const int n = min(tot - r0, kMaskStage);
+      if (tid == 0) { npair = 0; sharp_in = 0; }
+      if (f && pos >= r0 && pos < r0 + n) {
+        list[pos - r0] = p;
+      }
+      __syncthreads();
+      for (int e = tid; e < n * (int)(sizeof(Prim) / 16); e += NTHR) {
+        const int q = e / (int)(sizeof(Prim) / 16), w = e - q * (int)(sizeof(Prim) / 16);
+        reinterpret_cast<double2 *>(sp + q)[w] = reinterpret_cast<const double2 *>(prims + list[q])[w];
+      }
+      if (f && pos >= r0 && pos < r0 + n && type == PRIM_SHARP) sharp_in = 1;
+      __syncthreads();
+      // this wave's run of staged primitives
+      const int q0 = n * wv / WAVES, q1 = n * (wv + 1) / WAVES;
+      for (int q = q0; q < q1; ++q) {
+        const double x = prim_reach(sp[q], c, i, j, xi, yj);
+        val[q][lane] = x;
+        const unsigned long long hit = __ballot(x >= 0.0 && sp[q].type != PRIM_SHARP);
+        if (hit) {
+          int base = 0;
+          if (lane == 0) base = atomicAdd(&npair, __popcll(hit));
+          base = __builtin_amdgcn_readfirstlane(base);
+          if (hit >> lane & 1ull) pair[base + __popcll(hit & ((1ull << lane) - 1ull))] = (unsigned short)(q * kMaskPix + lane);
         }
-        const unsigned long long bal = __ballot(f);
-        const int cnt = __popcll(bal);
-        if (n + cnt > kMaskStage) {  // take the first kMaskStage - n of this group
-          const int take = kMaskStage - n;
-          const int pre = __popcll(bal & ((1ull << lane) - 1ull));
-          if (f && pre < take) list[n + pre] = p;
-          // resume after the last primitive taken
-          unsigned long long bb = bal;
-          int lastlane = -1;
-          for (int k = 0; k < take; ++k) {
-            lastlane = __ffsll((long long)bb) - 1;
-            bb &= bb - 1ull;
+      }
+      __syncthreads();
+      for (int k = tid; k < npair; k += NTHR) {
+        const int q = pair[k] / kMaskPix, l = pair[k] & (kMaskPix - 1);
+        val[q][l] = smooth_step(c, val[q][l], sp[q].type == PRIM_DOT ? sp[q].a[4] : c.t, c.h);
+      }
+      __syncthreads();
+      if (!sharp_in) {
+        double best = -1.0;
+        int bi = -1;
+        for (int q = q0; q < q1; ++q) {
+          const double v = val[q][lane];
+          if (v > best) { best = v; bi = q; }
+        }
+        rv[wv][lane] = best;
+        ri[wv][lane] = bi;
+        __syncthreads();
+        if (wv == 0) {
+          int w = -1;
+#pragma unroll
+          for (int k = 0; k < WAVES; ++k)
+            if (rv[k][lane] > m) { m = rv[k][lane]; w = ri[k][lane]; }
+          if (w >= 0) {
+            wi = list[w];
+            velocity(w);
           }
-          p0 = p0 + lastlane + 1;
-          n = kMaskStage;
-          break;
         }
-        if (f) list[n + __popcll(bal & ((1ull << lane) - 1ull))] = p;
-        n += cnt;
-        p0 += kMaskPix;
-      }
-      if (lane == 0) {
-        nstage = n;
-        pnext = p0 < np ? p0 : np;
-      }
-    }
-    __syncthreads();
-    // read once per pass: wave 0 rewrites both at the start of the next pass
-    const int n = nstage, pn = pnext;
-    if (n == 0) break;
-    for (int e = tid; e < n * (int)(sizeof(Prim) / 8); e += NTHR) {
-      const int q = e / (int)(sizeof(Prim) / 8), w = e - q * (int)(sizeof(Prim) / 8);
-      reinterpret_cast<double *>(sp + q)[w] = reinterpret_cast<const double *>(prims + list[q])[w];
-    }
-    __syncthreads();
-    for (int q = wv; q < n; q += WAVES) val[q][lane] = prim_value(sp[q], c, i, j, xi, yj);
-    __syncthreads();
-    if (wv == 0 && valid) {
-      for (int q = 0; q < n; ++q) {
-        const Prim &P = sp[q];
-        const double v = val[q][lane];
-        const double *a = P.a;
-        if (P.type == PRIM_SHARP) {
-          if (v > -1.5) {
+      } else if (wv == 0 && valid) {
+        for (int q = 0; q < n; ++q) {
+          const Prim &P = sp[q];
+          const double v = val[q][lane];
+          const double *a = P.a;
+          if (P.type == PRIM_SHARP) {
+            if (v > -1.5) {
+              m = v;
+              wi = list[q];
+              const double xs = xi * a[4] + yj * a[5];
+              if (xs - a[0] >= 2.0 * a[9]) { mvx = a[7]; mvy = a[8]; }
+            }
+          } else if (v > m) {
             m = v;
             wi = list[q];
-            const double xs = xi * a[4] + yj * a[5];
-            if (xs - a[0] >= 2.0 * a[9]) { mvx = a[7]; mvy = a[8]; }
-          }
-        } else if (v > m) {
-          m = v;
-          wi = list[q];
-          if (P.type == PRIM_SEG) {
-            const double xs = xi * a[4] - yj * a[5];
-            mvx = (a[7] + (xs - a[0]) * (a[9] - a[7]) / c.ds);
-            mvy = (a[8] + (xs - a[0]) * (a[10] - a[8]) / c.ds);
-          } else if (P.type == PRIM_HINGE) {
-            mvx = a[5]; mvy = a[6];
-          } else {
-            mvx = a[2]; mvy = a[3];
+            velocity(q);
           }
         }
       }
+      __syncthreads();  // the next round overwrites list, sp and val
     }
-    __syncthreads();  // the next pass overwrites list, sp and val
-    if (pn >= np) break;
+    __syncthreads();  // and the next group cnt
   }
   if (wv != 0 || !valid) return;
   if (c.vs4 || c.frame) {
