@@ -32,6 +32,7 @@
 #include "kernels_mask.hpp"
 #include "kernels_step.hpp"
 #include "kernels_fused.hpp"
+#include "transfer.hpp"
 #include "kernels_adjoint.hpp"
 #include "kinematics.hpp"
 #include "solid.hpp"
@@ -656,13 +657,12 @@ extern "C" int fsibe_dev_coftxy_noalloc(int nx, int ny, const double *d_f, doubl
 static int host_call(fsibe_spectral *c, const double *in, double *out, int kind, int which, double dt) {
   if (!c || !out || (kind != 3 && !in)) return set_err(FSIBE_EARG, "null argument");
   const size_t bytes = sizeof(double) * (size_t)c->nx * c->ny;
-  if (kind != 3) HIPCHK(hipMemcpyAsync(c->hbuf_in, in, bytes, hipMemcpyHostToDevice, c->stream));
+  if (kind != 3) HIPCHK(Transfer::get().upload(c->hbuf_in, in, bytes, c->stream));
   if (kind == 0) CHK(dev_coftxy(c, c->hbuf_in, c->hbuf_out, c->stream));
   else if (kind == 1) CHK(dev_cofitxy(c, c->hbuf_in, c->hbuf_out, c->stream));
   else if (kind == 2) CHK(dev_op(c, which, c->hbuf_in, c->hbuf_out, c->stream));
   else CHK(dev_vis(c, dt, c->hbuf_out, c->stream));
-  HIPCHK(hipMemcpyAsync(out, c->hbuf_out, bytes, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(Transfer::get().download(out, c->hbuf_out, bytes, c->stream));
   return FSIBE_OK;
 }
 
@@ -1660,7 +1660,7 @@ extern "C" int fsibe_sim_create(const fsibe_params *pp, fsibe_sim **out) {
 extern "C" int fsibe_set_vortk(fsibe_sim *s, const double *vk) {
   if (!s || !vk) return set_err(FSIBE_EARG, "null argument");
   const size_t N = (size_t)s->nx * s->ny;
-  HIPCHK(hipMemcpyAsync(s->fb_p, vk, sizeof(double) * N, hipMemcpyHostToDevice, s->stream));
+  HIPCHK(Transfer::get().upload(s->fb_p, vk, sizeof(double) * N, s->stream));
   k_packed_to_half<<<grid1d((size_t)s->H * (s->ny / 2)), 256, 0, s->stream>>>(s->fb_p, s->W[s->n0], s->nx, s->ny);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s->stream));
@@ -2937,17 +2937,17 @@ extern "C" int fsibe_get_field(fsibe_sim *s, int which, double *out) {
       const double2 *src = which == FSIBE_FIELD_VORTK ? s->W[s->n0] : s->NL[s->n0];
       k_half_to_packed<<<g, 256, 0, s->stream>>>(src, s->fb_p, s->nx, s->ny);
       HIPCHK(hipGetLastError());
-      HIPCHK(hipMemcpyAsync(out, s->fb_p, sizeof(double) * N, hipMemcpyDeviceToHost, s->stream));
+      HIPCHK(Transfer::get().download(out, s->fb_p, sizeof(double) * N, s->stream));
       s->press_box_valid = false;
       break;
     }
-    case FSIBE_FIELD_U1: HIPCHK(hipMemcpyAsync(out, s->u1, sizeof(double) * N, hipMemcpyDeviceToHost, s->stream)); break;
-    case FSIBE_FIELD_U2: HIPCHK(hipMemcpyAsync(out, s->u2, sizeof(double) * N, hipMemcpyDeviceToHost, s->stream)); break;
+    case FSIBE_FIELD_U1: HIPCHK(Transfer::get().download(out, s->u1, sizeof(double) * N, s->stream)); break;
+    case FSIBE_FIELD_U2: HIPCHK(Transfer::get().download(out, s->u2, sizeof(double) * N, s->stream)); break;
     case FSIBE_FIELD_VOR_MEAN:
-      HIPCHK(hipMemcpyAsync(out, s->vor_mean, sizeof(double) * N, hipMemcpyDeviceToHost, s->stream));
+      HIPCHK(Transfer::get().download(out, s->vor_mean, sizeof(double) * N, s->stream));
       break;
     case FSIBE_FIELD_MASK_SPONGE:
-      if (s->ms) HIPCHK(hipMemcpyAsync(out, s->ms, sizeof(double) * N, hipMemcpyDeviceToHost, s->stream));
+      if (s->ms) HIPCHK(Transfer::get().download(out, s->ms, sizeof(double) * N, s->stream));
       else memset(out, 0, sizeof(double) * N);
       break;
     case FSIBE_FIELD_MASK: return box_to_full(s, s->mask_m, s->mbox, out);
@@ -2958,7 +2958,7 @@ extern "C" int fsibe_get_field(fsibe_sim *s, int which, double *out) {
       const int fsel[1] = {0};
       CHK(cols_inv_fields(s, s->W[s->n0], outs, fsel, 1));
       CHK(rows_c2r(s->nx, s->ny, s->px, s->twx, s->T[6], s->fb_sb, s->stream));
-      HIPCHK(hipMemcpyAsync(out, s->fb_sb, sizeof(double) * N, hipMemcpyDeviceToHost, s->stream));
+      HIPCHK(Transfer::get().download(out, s->fb_sb, sizeof(double) * N, s->stream));
       s->press_box_valid = false;
       break;
     }
@@ -2977,7 +2977,7 @@ extern "C" int fsibe_get_field(fsibe_sim *s, int which, double *out) {
                 s->u2, s->fb_sb, s->fb_sa, s->fb_sa, 0, 0, s->nx - 1, s->nx, 0, F, s->twx, s->sc);
         return FSIBE_OK;
       }));
-      HIPCHK(hipMemcpyAsync(out, s->fb_sb, sizeof(double) * N, hipMemcpyDeviceToHost, s->stream));
+      HIPCHK(Transfer::get().download(out, s->fb_sb, sizeof(double) * N, s->stream));
       s->press_box_valid = false;
       break;
     }

@@ -1,17 +1,19 @@
-// transfer.hpp -- copies between a caller's pageable host memory and the GPU.
+// transfer.hpp -- large copies between a caller's pageable host memory and the
+// GPU.
 //
 // The runtime's own copy of pageable memory stages it through its pinned
 // buffers with one host thread: about 6 GB/s for a field read into fresh
 // memory, whose pages that thread also faults in (134 MB, a 4096^2 field:
 // 22 ms, as long as 20 of its time steps).  Here the copy engine moves
-// chunks between the device and a pinned ring while a few host threads move
-// them between the ring and the caller's memory.
+// chunks between the device and a pinned ring while a few host threads, each
+// a chunk at a time, move them between the ring and the caller's memory.
 //
 // One ring and one pool of threads per process, made at the first large
-// copy: at most 16 MiB pinned and 7 threads, asleep between copies.  A copy
+// copy: 32 MiB pinned and at most 7 threads, asleep between copies.  A copy
 // that finds them in use by another thread, or whose host pointer the runtime
 // already knows (pinned, managed or device memory), takes the runtime's path,
-// as does a small one.
+// as does one of less than 4 MiB (1.2 MB: 90 us by the runtime, 180 us here,
+// where waking the threads and a call per chunk cost more than they save).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <unistd.h>
@@ -19,6 +21,7 @@
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
+#include <cstdint>
 #include <cstring>
 #include <mutex>
 #include <thread>
@@ -52,10 +55,9 @@ class Transfer {
   }
 
  private:
-  static constexpr size_t kMin = 192 << 10;   // below, the runtime's path is as fast
-  static constexpr size_t kUnit = 64 << 10;   // one host copy
-  static constexpr size_t kSlot = 2 << 20;    // largest chunk (one device copy)
-  static constexpr int kSlots = 8, kHelpers = 7;
+  static constexpr size_t kMin = 4 << 20;
+  static constexpr size_t kSlot = 2 << 20;  // largest chunk: a huge page, faulted in by one thread
+  static constexpr int kSlots = 16, kHelpers = 7;
 
   hipError_t plain(void *dst, const void *src, size_t bytes, hipStream_t st, bool up) {
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, st);
@@ -97,63 +99,78 @@ class Transfer {
     if (known == hipSuccess && at.type != hipMemoryTypeUnregistered) return plain(dst, src, bytes, st, up);
     std::unique_lock<std::mutex> use(use_, std::try_to_lock);
     if (!use.owns_lock() || !ready()) return plain(dst, src, bytes, st, up);
-    // about six chunks of a small copy, so that both halves of the way are busy
-    const size_t chunk = std::min(kSlot, std::max((bytes / 6 + kUnit - 1) / kUnit, (size_t)2) * kUnit);
-    const long n = (long)((bytes + chunk - 1) / chunk);
-    const int slots = (int)std::min<long>(n, kSlots);
+    Job j;
+    j.host = up ? (char *)const_cast<void *>(src) : (char *)dst;
+    j.dev = up ? (char *)dst : (char *)const_cast<void *>(src);
+    j.bytes = bytes;
+    j.chunk = std::min(kSlot, std::max(bytes / 12 >> 16 << 16, (size_t)512 << 10));
+    // the first chunk ends where the others are aligned
+    j.lead = j.chunk - (size_t)((uintptr_t)j.host % j.chunk);
+    j.n = 1 + (long)((bytes - std::min(bytes, j.lead) + j.chunk - 1) / j.chunk);
+    j.up = up;
+    const int slots = (int)std::min<long>(j.n, kSlots);
     hipEvent_t ev[kSlots];
     int nev = 0;
     hipError_t e = hipSuccess;
     while (nev < slots && e == hipSuccess)
       if ((e = hipEventCreateWithFlags(&ev[nev], hipEventDisableTiming)) == hipSuccess) ++nev;
     if (e == hipSuccess) {
-      auto len = [&](long i) { return std::min(chunk, bytes - (size_t)i * chunk); };
-      auto slot = [&](long i) { return ring_ + (size_t)(i % kSlots) * kSlot; };
-      start(Job{up ? (char *)const_cast<void *>(src) : (char *)dst, bytes, chunk, up});
-      if (up) {
-        for (long i = 0; i < n && e == hipSuccess; ++i) {
-          if (i >= kSlots) e = hipEventSynchronize(ev[i % kSlots]);  // the slot's last chunk is on the device
-          if (e != hipSuccess) break;
-          move_chunk(i);
-          e = hipMemcpyAsync((char *)dst + (size_t)i * chunk, slot(i), len(i), hipMemcpyHostToDevice, st);
-          if (e == hipSuccess) e = hipEventRecord(ev[i % kSlots], st);
+      start(j);
+      // chunk i uses slot i % kSlots once chunk i - kSlots has left it
+      long issued = 0, ready = 0;  // device copies issued; chunks the helpers may move
+      auto moved = [&](long i) { return slot_done_[i % kSlots].load(std::memory_order_acquire) >= i + 1; };
+      auto landed = [&](long i) {  // chunk i's device copy is over (or has failed: e)
+        const hipError_t q = hipEventQuery(ev[i % kSlots]);
+        if (q != hipSuccess && q != hipErrorNotReady) e = q;
+        return q == hipSuccess;
+      };
+      auto issue = [&](long i) {
+        char *r = ring_ + (size_t)(i % kSlots) * kSlot, *d = j.dev + j.begin(i);
+        e = up ? hipMemcpyAsync(d, r, j.len(i), hipMemcpyHostToDevice, st)
+               : hipMemcpyAsync(r, d, j.len(i), hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipEventRecord(ev[i % kSlots], st);
+      };
+      while (e == hipSuccess && (up ? issued : ready) < j.n) {
+        bool any = false;
+        if (up) {
+          if (ready < j.n && (ready < kSlots || (ready - kSlots < issued && landed(ready - kSlots)))) ++ready, any = true;
+          if (issued < ready && moved(issued)) issue(issued++), any = true;
+        } else {
+          if (issued < j.n && (issued < kSlots || moved(issued - kSlots))) issue(issued++), any = true;
+          if (e == hipSuccess && ready < issued && landed(ready)) ++ready, any = true;
         }
-      } else {
-        long issued = 0;
-        for (long i = 0; i < n && e == hipSuccess; ++i) {
-          // chunk issued - kSlots has left its slot: move_chunk returned for it
-          for (; issued < n && issued < i + kSlots && e == hipSuccess; ++issued) {
-            e = hipMemcpyAsync(slot(issued), (const char *)src + (size_t)issued * chunk, len(issued),
-                               hipMemcpyDeviceToHost, st);
-            if (e == hipSuccess) e = hipEventRecord(ev[issued % kSlots], st);
-          }
-          if (e == hipSuccess) e = hipEventSynchronize(ev[i % kSlots]);
-          if (e == hipSuccess) move_chunk(i);
-        }
+        if (any) published_.store(ready, std::memory_order_release);
+        else if (!workers_.empty() || !help()) std::this_thread::yield();
       }
+      if (e == hipSuccess && !up)
+        for (long i = std::max(0L, j.n - kSlots); i < j.n; ++i)
+          while (!moved(i))
+            if (!help()) std::this_thread::yield();
       end();
       // no device copy from or into the ring outlives the call
-      const hipError_t s = hipStreamSynchronize(st);
-      if (e == hipSuccess) e = s;
+      const hipError_t q = hipStreamSynchronize(st);
+      if (e == hipSuccess) e = q;
     }
     for (int i = 0; i < nev; ++i) (void)hipEventDestroy(ev[i]);
+    if (e == hipSuccess) (void)hipGetLastError();  // an event query's "not ready" is no error of the caller's
     return e;
   }
 
-  // ---- host copies: units of a chunk, taken by whoever is free
+  // ---- host copies: a chunk at a time, taken by whoever is free
   struct Job {
-    char *host;
-    size_t bytes, chunk;
+    char *host, *dev;
+    size_t bytes, chunk, lead;
+    long n;
     bool up;
-    long units() const { return (long)((bytes + kUnit - 1) / kUnit); }
-    long per_chunk() const { return (long)(chunk / kUnit); }
+    size_t begin(long i) const { return i == 0 ? 0 : std::min(bytes, lead + (size_t)(i - 1) * chunk); }
+    size_t len(long i) const { return begin(i + 1) - begin(i); }
   };
   void start(const Job &j) {
     job_ = j;
     published_.store(0);
     next_.store(0);
-    moved_.store(0);
     over_.store(false);
+    for (auto &d : slot_done_) d.store(0);
     {
       std::lock_guard<std::mutex> g(mu_);
       active_ = (int)workers_.size();
@@ -161,26 +178,17 @@ class Transfer {
     }
     cv_.notify_all();
   }
-  void move_unit(long u) {
-    const size_t off = (size_t)u * kUnit, len = std::min(kUnit, job_.bytes - off);
-    const long i = u / job_.per_chunk();
-    char *h = job_.host + off, *r = ring_ + (size_t)(i % kSlots) * kSlot + (off - (size_t)i * job_.chunk);
-    if (job_.up) memcpy(r, h, len);
-    else memcpy(h, r, len);
-    moved_.fetch_add(1, std::memory_order_acq_rel);
-  }
-  // lets the helpers at chunk i (its slot is ready), takes part, and returns
-  // when all units of chunks 0 .. i have been moved (no later unit can have been)
-  void move_chunk(long i) {
-    const long want = std::min((i + 1) * job_.per_chunk(), job_.units());
-    published_.store(want, std::memory_order_release);
-    long u = next_.load();
-    while (u < want)
-      if (next_.compare_exchange_weak(u, u + 1)) {
-        move_unit(u);
-        u = next_.load();
-      }
-    while (moved_.load(std::memory_order_acquire) < want) std::this_thread::yield();
+  // moves the next published chunk; false if there is none
+  bool help() {
+    long i = next_.load();
+    do {
+      if (i >= published_.load(std::memory_order_acquire)) return false;
+    } while (!next_.compare_exchange_weak(i, i + 1));
+    char *h = job_.host + job_.begin(i), *r = ring_ + (size_t)(i % kSlots) * kSlot;
+    if (job_.up) memcpy(r, h, job_.len(i));
+    else memcpy(h, r, job_.len(i));
+    slot_done_[i % kSlots].store(i + 1, std::memory_order_release);
+    return true;
   }
   void end() {
     over_.store(true, std::memory_order_release);
@@ -196,17 +204,9 @@ class Transfer {
         if (stop_) return;
         seen = gen_;
       }
-      const long n = job_.units();
-      for (;;) {
-        if (over_.load(std::memory_order_acquire)) break;  // nothing left, or the copy failed
-        long u = next_.load();
-        if (u >= n) break;
-        if (u < published_.load(std::memory_order_acquire)) {
-          if (next_.compare_exchange_weak(u, u + 1)) move_unit(u);
-        } else {
-          std::this_thread::yield();
-        }
-      }
+      // until all chunks are taken, or the copy failed
+      while (!over_.load(std::memory_order_acquire) && next_.load() < job_.n)
+        if (!help()) std::this_thread::yield();
       std::lock_guard<std::mutex> g(mu_);
       if (--active_ == 0) done_.notify_one();
     }
@@ -221,7 +221,8 @@ class Transfer {
   unsigned long long gen_ = 0;
   int active_ = 0;
   Job job_{};
-  std::atomic<long> published_{0}, next_{0}, moved_{0};
+  std::atomic<long> published_{0}, next_{0};
+  std::atomic<long> slot_done_[kSlots] = {};  // 1 + the last chunk moved through the slot
   std::atomic<bool> over_{false};
 };
 
