@@ -397,6 +397,27 @@ static bool with_col_step(int ny, int H, bool px, Fn &&fn) {
   }
 }
 
+// fn(shape) for the pressure stage (K7) of columns of ny values; false if
+// there is none (odd H, other lengths, and columns whose two buffers leave
+// one workgroup on a CU)
+template <class Fn>
+static bool with_press_step(int ny, int H, Fn &&fn) {
+  if (H % 2) return false;
+  switch (ny) {
+    case 64: fn(PressShape<64, 2, 8>{}); return true;
+    case 96: fn(PressShape<96, 2, 12>{}); return true;
+    case 128: fn(PressShape<128, 2, 16>{}); return true;
+    case 192: fn(PressShape<192, 2, 24>{}); return true;
+    case 256: fn(PressShape<256, 2, 32>{}); return true;
+    case 384: fn(PressShape<384, 2, 48>{}); return true;
+    case 512: fn(PressShape<512, 2, 64>{}); return true;
+    case 768: fn(PressShape<768, 2, 96>{}); return true;
+    case 1024: fn(PressShape<1024, 2, 128>{}); return true;
+    case 1536: fn(PressShape<1536, 2, 192>{}); return true;
+    default: return false;
+  }
+}
+
 // transform lengths that a policy fixes at compile time (0: a runtime plan),
 // so that the fallbacks below are not instantiated where they cannot run
 template <class F> struct fixed_len { static constexpr int v = 0; };
@@ -2408,6 +2429,27 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
   return FSIBE_OK;
 }
 
+// K7: the inverse column transform of the pressure (T4, T5) on rows r0 .. r1, into T6
+static int launch_press(fsibe_sim *s, int r0, int r1) {
+  int rc = FSIBE_OK;
+  const bool fast = with_press_step(s->ny, s->H, [&](auto S) {
+    using ST = decltype(S);
+    PressArgs a;
+    a.Rq = s->T[4]; a.Rqy = s->T[5]; a.Cq = s->T[6]; a.r0 = r0; a.r1 = r1; a.c = s->sc;
+    rc = [&]() -> int {
+      KLAUNCH(k_press_step<ST>, s->H / ST::TX, ST::THREADS, ST::LDS, s->stream, a, s->twy);
+      return FSIBE_OK;
+    }();
+  });
+  if (fast) return rc;
+  return with_cols_sel<2>(s->py, s->H, sim_sel(s, 3, 1), [&](auto F, int nt, int TX) -> int {
+    const size_t lds = sizeof(double2) * 2 * TX * padlen(s->ny);
+    KLAUNCH(k_cols_press<decltype(F)>, s->H / TX, nt, lds, s->stream, s->T[4], s->T[5], s->T[6], r0, r1, F, s->twy,
+            s->sc);
+    return FSIBE_OK;
+  });
+}
+
 // K7 + K8: the static pressure and the stresses on the rows/columns the
 // interpolation needs (the box of the force geometry)
 static int evolve_pressure_box(fsibe_sim *s) {
@@ -2416,12 +2458,7 @@ static int evolve_pressure_box(fsibe_sim *s) {
     const Box &fb = s->fbox;
     {
       PROF_BEGIN(s, P_COLS_PRESS);
-      CHK(with_cols_sel<2>(s->py, s->H, sim_sel(s, 3, 1), [&](auto F, int nt, int TX) -> int {
-        const size_t lds = sizeof(double2) * 2 * TX * padlen(s->ny);
-        KLAUNCH(k_cols_press<decltype(F)>, s->H / TX, nt, lds, s->stream, s->T[4], s->T[5], s->T[6], fb.y0, fb.y1,
-                F, s->twy, s->sc);
-        return FSIBE_OK;
-      }));
+      CHK(launch_press(s, fb.y0, fb.y1));
       prof_end(s, P_COLS_PRESS);
     }
     {
@@ -2965,12 +3002,7 @@ extern "C" int fsibe_get_field(fsibe_sim *s, int which, double *out) {
     case FSIBE_FIELD_PRESS: {
       if (!s->pressure_on) { memset(out, 0, sizeof(double) * N); break; }
       // full-grid pressure from the last step's right-hand side (T4, T5)
-      CHK(with_cols_sel<2>(s->py, s->H, sim_sel(s, 3, 1), [&](auto F, int nt, int TX) -> int {
-        const size_t lds = sizeof(double2) * 2 * TX * padlen(s->ny);
-        KLAUNCH(k_cols_press<decltype(F)>, s->H / TX, nt, lds, s->stream, s->T[4], s->T[5], s->T[6], 0, s->ny - 1,
-                F, s->twy, s->sc);
-        return FSIBE_OK;
-      }));
+      CHK(launch_press(s, 0, s->ny - 1));
       const size_t lds2 = sizeof(double2) * 3 * padlen(s->H);
       CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
         KLAUNCH(k_rows_box<decltype(F)>, s->ny, nt, lds2, s->stream, s->T[6], s->T[1], s->T[2], s->T[3], s->u1,

@@ -455,6 +455,93 @@ __global__ void __launch_bounds__(S::THREADS) kb_col_step(const ColStepRec *__re
 }
 
 // ============================================================================
+// Pressure stage (K7)
+// ============================================================================
+struct PressArgs {
+  const double2 *Rq, *Rqy;
+  double2 *Cq;
+  int r0, r1;  // rows of the inverse transform that are stored
+  StepConsts c;
+};
+
+// the spectrum of q at mode (kx, idx) from the transforms of the two
+// right-hand sides (pressure, NavierStokes.f90:366-382)
+template <int L>
+__device__ __forceinline__ double2 press_mode(const StepConsts &c, int kx, int idx, double2 a, double2 b) {
+  const int ky = ky_signed(idx, L);
+  const int aky = ky < 0 ? -ky : ky;
+  if (idx == L / 2 || (kx == 0 && ky == 0)) return make_double2(0.0, 0.0);
+  const double kyf = (double)ky * c.sy;
+  const double2 fa = make_double2(a.x * c.norm, a.y * c.norm);
+  const double2 fb = make_double2(b.x * c.norm, b.y * c.norm);
+  const double2 rhs = make_double2(fa.x - kyf * fb.y, fa.y + kyf * fb.x);
+  const double quot = ((double)(kx * kx) * c.scalex + (double)(aky * aky) * c.scaley), rq = 1.0 / quot;
+  return make_double2(div_by(rhs.x, quot, rq), div_by(rhs.y, quot, rq));
+}
+
+// Two slots of TX*NT threads transform one right-hand side each straight from
+// memory, all threads form q, slot 0 transforms it back into memory.  It
+// reads two fields and stores a band of rows: bound by memory from about
+// 1024^2, by the chain of two transforms below.  Against the stage that
+// staged its columns in LDS first (compile-time plan, best width): 5.8 -> 5.1
+// us at 256^2, 6.6 -> 5.5 at 512^2, 11.0 -> 9.3 at 1024^2, 19.8 -> 14.5 at
+// 1024 x 1536.  Two columns per workgroup: one gives 5.1, 6.1, 11.3, 16.1 us.
+template <int L, int TX, int NT>
+__device__ __forceinline__ void press_step_body(const PressArgs &a, const double2 *__restrict__ twy, int bid, int nblk) {
+  extern __shared__ double2 lds[];
+  constexpr int PL = padlen(L), NTHR = 2 * TX * NT, SB = TX * PL;
+  constexpr bool WAVE = NTHR <= 64;
+  using Out = FftOut<L, NT>;
+  const StepConsts &c = a.c;
+  const int tid = threadIdx.x, H = c.H;
+  const int slot = tid / (TX * NT), w = tid - slot * (TX * NT), cc = w % TX, t = w / TX;
+  const int kx0 = xcd_remap(bid, nblk) * TX;
+  double2 *xb = lds + slot * SB + cc;
+  FftTw<L, NT> T;
+  T.load(twy, 1, t);
+  {
+    double2 z[Out::N];
+    const double2 *src = (slot == 0 ? a.Rq : a.Rqy) + kx0 + cc;
+    fft_io<L, NT, false, TX, WAVE, false>(
+        xb, T, t, true, [&](int, int, int e) { return src[(size_t)e * H]; },
+        [&](int i, int r, int, double2 x) { z[i * Out::R + r] = x; });
+    grp_sync<WAVE>();
+#pragma unroll
+    for (int i = 0; i < Out::ITEMS; ++i) {
+      const int j = t + i * NT;
+      if (Out::M % NT == 0 || j < Out::M) {
+#pragma unroll
+        for (int r = 0; r < Out::R; ++r) xb[pidx(j + r * Out::M) * TX] = z[i * Out::R + r];
+      }
+    }
+    grp_sync<WAVE>();
+  }
+  for (int e = tid; e < L * TX; e += NTHR) {
+    const int idx = e / TX, c2 = e % TX;
+    double2 *l0 = lds + pidx(idx) * TX + c2;
+    *l0 = press_mode<L>(c, kx0 + c2, idx, l0[0], l0[SB]);
+  }
+  grp_sync<WAVE>();
+  fft_io<L, NT, true, TX, WAVE, false>(
+      xb, T, t, slot == 0, [&](int, int, int e) { return xb[pidx(e) * TX]; },
+      [&](int, int, int e, double2 x) {
+        if (e >= a.r0 && e <= a.r1) a.Cq[(size_t)e * H + kx0 + cc] = x;
+      });
+}
+
+template <int LC, int TXC, int NTC> struct PressShape {
+  static constexpr int L = LC, TX = TXC, NT = NTC, THREADS = 2 * TX * NT;
+  static constexpr size_t LDS = sizeof(double2) * 2 * TX * padlen(L);
+  static __device__ __forceinline__ void run(const PressArgs &a, const double2 *__restrict__ twy, int bid, int nblk) {
+    press_step_body<L, TX, NT>(a, twy, bid, nblk);
+  }
+};
+template <class S>
+__global__ void __launch_bounds__(S::THREADS) k_press_step(PressArgs a, const double2 *__restrict__ twy) {
+  S::run(a, twy, blockIdx.x, gridDim.x);
+}
+
+// ============================================================================
 // Row stage
 // ============================================================================
 struct RowStepArgs {

@@ -51,3 +51,26 @@ def test_one_call_of_several_steps_equals_several_calls_of_one(nx, ny, kind):
     for k in ("dt1", "u_max", "Force", "Force_press", "energies", "bsi"):
         assert oa[k] == ob[k], k
     assert np.array_equal(ba["pressure"], bb["pressure"]) and np.array_equal(ba["tau"], bb["tau"])
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 64), (128, 96), (64, 128), (108, 192), (256, 256), (128, 384), (192, 512),
+                                   (256, 768), (128, 1024), (64, 1536)])
+def test_pressure_stage_equals_the_batched_one(nx, ny):
+    """the single path's pressure stage (two slots per column) against the
+    batch's (columns staged in LDS): the same operations, so the loads agree
+    bit for bit; 108 x 192 has an odd number of columns and shares the code"""
+    from fsibe_2d_amd import Params
+    from fsibe_2d_amd.solver import Batch, FluidSim
+
+    p = Params(nx=nx, ny=ny, ns=33, nu=2e-3, dt_fixed=2e-4)
+    b = Batch([p], [None])
+    b.run(3)
+    s = FluidSim(p)
+    out, want = s.run(3), b.members[0].step_out()
+    for k in ("Force_press", "bsi"):
+        assert out[k] == want[k], k
+    for k in ("pressure", "tau"):
+        assert np.array_equal(s.beam()[k], b.members[0].beam()[k]), k
+    assert np.abs(s.beam()["pressure"]).max() > 0.0
+    s.close()
+    b.close()
