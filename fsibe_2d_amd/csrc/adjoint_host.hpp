@@ -22,24 +22,29 @@ static void adj_copy_d(hipStream_t st, const double *src, double *dst, size_t n)
   const int blocks = (int)std::min<size_t>(1024, (n + 255) / 256);
   ak_copy_d<<<blocks, 256, 0, st>>>(src, dst, (long long)n);
 }
-static void adj_copy_i(hipStream_t st, const int *src, int *dst, size_t n) {
-  if (n == 0) return;
-  const int blocks = (int)std::min<size_t>(1024, (n + 255) / 256);
-  ak_copy_i<<<blocks, 256, 0, st>>>(src, dst, (long long)n);
-}
 static void adj_zero(hipStream_t st, double *dst, size_t n) {
   if (n == 0) return;
   const int blocks = (int)std::min<size_t>(1024, (n + 255) / 256);
   ak_zero<<<blocks, 256, 0, st>>>(dst, (long long)n);
 }
 
+// The steps of a unit leave what the adjoint needs in the tape's slots as
+// they compute it: while a unit is recorded the simulation's mask, velocity
+// and the columns A, B of its nonlinear term are the current step's slots
+// (the pointers below hold its own buffers meanwhile).  Copying them
+// afterwards took eight more launches a step, 20 us of a 512^2 step's 75.
 struct AdjTape {
-  int cap = 0, n = 0;
+  int cap = 0, n = 0, len = 0;  // slots, steps recorded, steps of the unit
   size_t NH = 0, N = 0;
   double2 *A = nullptr, *B = nullptr;
   double *u1 = nullptr, *u2 = nullptr, *m = nullptr, *vx = nullptr, *vy = nullptr;
   int *win = nullptr;
   DevScalars *sc = nullptr;
+  struct Own {
+    double2 *T0, *T1, *T7;
+    double *u1, *u2, *m, *vx, *vy;
+    int *win;
+  } own{};
   struct Rec {
     Box mbox;
     Window win;
@@ -49,40 +54,73 @@ struct AdjTape {
   std::vector<Rec> rec;
 };
 
-// after create_mask: the mask box (values, velocities, winning primitives),
-// the cal_drag window and the time of the kinematics the beam arrays hold
+static void tape_begin(fsibe_sim *s, AdjTape &t, int len) {
+  t.n = 0;
+  t.len = len;
+  t.own = AdjTape::Own{s->T[0], s->T[1], s->T[7], s->u1, s->u2, s->mask_m, s->mask_vx, s->mask_vy, s->mask_win};
+  s->tape = &t;
+}
+static void tape_end(fsibe_sim *s) {
+  const AdjTape::Own &o = s->tape->own;
+  s->T[0] = o.T0; s->T[1] = o.T1; s->T[7] = o.T7;
+  s->u1 = o.u1; s->u2 = o.u2;
+  s->mask_m = o.m; s->mask_vx = o.vx; s->mask_vy = o.vy; s->mask_win = o.win;
+  s->tape = nullptr;
+}
+
+// before the mask kernel: its outputs are the step's slot
+static void tape_mask_place(fsibe_sim *s) {
+  AdjTape &t = *s->tape;
+  if (t.n >= t.cap) return;
+  const size_t o = (size_t)t.n * t.N;
+  s->mask_m = t.m + o; s->mask_vx = t.vx + o; s->mask_vy = t.vy + o;
+  if (s->mask_win) s->mask_win = t.win + o;
+}
+
+// after create_mask: the mask box, the cal_drag window and the time of the
+// kinematics the beam arrays hold
 static void tape_mask(fsibe_sim *s) {
   AdjTape &t = *s->tape;
   if (t.n >= t.cap) return;
-  const int j = t.n;
-  AdjTape::Rec &r = t.rec[j];
+  AdjTape::Rec &r = t.rec[t.n];
   r.mbox = s->mbox;
   r.win = s->win[0];  // one beam: the adjoint runs iBeam = 1 only
   r.tau = s->beam_time;
-  const size_t nb = s->mbox.empty() ? 0 : (size_t)s->mbox.w() * s->mbox.h();
-  adj_copy_d(s->stream, s->mask_m, t.m + j * t.N, nb);
-  adj_copy_d(s->stream, s->mask_vx, t.vx + j * t.N, nb);
-  adj_copy_d(s->stream, s->mask_vy, t.vy + j * t.N, nb);
-  if (s->mask_win) adj_copy_i(s->stream, s->mask_win, t.win + j * t.N, nb);
 }
 
-// after the nonlinear-term kernel: A, B (its column inputs), u of this step
-// (it is overwritten by the velocity kernel) and the step's scalars
+// before K1: its columns A, B are the step's slot
+static void tape_k1_place(fsibe_sim *s) {
+  AdjTape &t = *s->tape;
+  if (t.n >= t.cap) return;
+  s->T[0] = t.A + (size_t)t.n * t.NH;
+  s->T[1] = t.B + (size_t)t.n * t.NH;
+}
+
+// after the nonlinear-term kernel: A, B (its column inputs) and u of this
+// step are in its slot but for the unit's first velocity; the step's scalars
+// are copied; what the rest of the step forms for the next one (its columns
+// A, B and its velocity) goes to the next slot
 static int tape_fluid(fsibe_sim *s, bool explicit_step) {
   AdjTape &t = *s->tape;
   if (t.n >= t.cap) return set_err(FSIBE_ESTATE, "adjoint tape full");
-  const int j = t.n;
-  adj_copy_d(s->stream, reinterpret_cast<const double *>(s->T[0]), reinterpret_cast<double *>(t.A + j * t.NH),
-             2 * t.NH);
-  adj_copy_d(s->stream, reinterpret_cast<const double *>(s->Bp), reinterpret_cast<double *>(t.B + j * t.NH),
-             2 * t.NH);
-  adj_copy_d(s->stream, s->u1, t.u1 + j * t.N, t.N);
-  adj_copy_d(s->stream, s->u2, t.u2 + j * t.N, t.N);
+  const size_t j = t.n;
+  if (s->T[0] != t.A + j * t.NH || s->Bp != t.B + j * t.NH)
+    return set_err(FSIBE_ESTATE, "adjoint: the columns of step %d are not on the tape", t.n);
+  if (s->u1 != t.u1 + j * t.N) {
+    adj_copy_d(s->stream, s->u1, t.u1 + j * t.N, t.N);
+    adj_copy_d(s->stream, s->u2, t.u2 + j * t.N, t.N);
+  }
   adj_copy_d(s->stream, reinterpret_cast<const double *>(s->dscal), reinterpret_cast<double *>(t.sc + j),
              sizeof(DevScalars) / sizeof(double));
   HIPCHK(hipGetLastError());
+  const bool more = t.n + 1 < t.len;
+  s->T[0] = more ? t.A + (j + 1) * t.NH : t.own.T0;
+  s->T[7] = more ? t.B + (j + 1) * t.NH : t.own.T7;
+  s->T[1] = t.own.T1;
+  s->u1 = more ? t.u1 + (j + 1) * t.N : t.own.u1;
+  s->u2 = more ? t.u2 + (j + 1) * t.N : t.own.u2;
   t.rec[j].explicit_step = explicit_step ? 1 : 0;
-  t.n = j + 1;
+  t.n = (int)j + 1;
   return FSIBE_OK;
 }
 
@@ -461,9 +499,6 @@ static int adj_reverse_step(fsibe_adjoint *a, int j, const double *u1n, double c
   mb.m = t.m + j * t.N; mb.vx = t.vx + j * t.N; mb.vy = t.vy + j * t.N;
   double2 *Ta = a->T[0], *Tb = a->T[1], *Tc = a->T[2], *Td = a->T[3], *Te = a->T[4], *Tf = a->T[5];
   const size_t nbox = r.mbox.empty() ? 0 : (size_t)r.mbox.w() * r.mbox.h();
-  adj_zero(s->stream, a->lm, nbox);
-  adj_zero(s->stream, a->lvx, nbox);
-  adj_zero(s->stream, a->lvy, nbox);
   CHK(with_rows<2>(s->px, [&](auto F, int nt) -> int {
     KLAUNCH(ak_rows_vel<decltype(F)>, s->ny, nt, sizeof(double2) * 2 * padlen(s->H), s->stream, a->lu1, a->lu2,
             u1n, mb, r.win, cJ, a->lm, a->lvx, a->lvy, Ta, Tb, F, s->twx, s->sc);
@@ -514,8 +549,7 @@ static int adj_record_reverse(fsibe_adjoint *a, int k, double *J, double *T, dou
   fsibe_sim *s = a->s;
   const int first = unit_start(a, k), len = unit_start(a, k + 1) - first;
   AdjTape &t = a->tape;
-  t.n = 0;
-  s->tape = &t;
+  tape_begin(s, t, len);
   int rc = FSIBE_OK;
   // pipelined as fsibe_run's prescribed-motion loop: the host prepares
   // step j+1 while step j runs and reads each step's results one step late
@@ -529,7 +563,7 @@ static int adj_record_reverse(fsibe_adjoint *a, int k, double *J, double *T, dou
                      first + j, s->dt1);
     }
   }
-  s->tape = nullptr;
+  tape_end(s);
   s->pipe = false;
   s->k1_ready = false;
   s->k2_ready = false;

@@ -1131,6 +1131,8 @@ struct fsibe_sim {
   struct AdjTape *tape = nullptr;  // records the forward data of each step for the adjoint
 };
 
+static void tape_mask_place(fsibe_sim *s);
+static void tape_k1_place(fsibe_sim *s);
 static void tape_mask(fsibe_sim *s);
 static int tape_fluid(fsibe_sim *s, bool explicit_step);
 
@@ -2097,6 +2099,7 @@ static int create_mask_impl(fsibe_sim *s, double time, const double *x, const do
   }
   CHK(upload_geometry(s));
   prof_host(s, P_REDUCE, th0);
+  if (s->tape) tape_mask_place(s);
   if (!s->mbox.empty()) {
     MaskConsts mc;
     mc.dx = s->dx; mc.dy = s->dy; mc.t = s->p.t_beam; mc.h = s->p.N_smooth * std::max(s->dx, s->dy);
@@ -2281,6 +2284,7 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
     s->k1_ready = false;  // K1 of this step was launched ahead (run_one)
   } else {
     s->k1_ready = false;
+    if (s->tape) tape_k1_place(s);
     CHK(launch_k1(s, n0));
   }
   MaskBox mb = mask_box(s);

@@ -363,12 +363,8 @@ __global__ void __launch_bounds__(256) ak_mask(const int *__restrict__ win, cons
   }
 }
 
-// device-to-device copies of n doubles / ints (tape and checkpoints)
+// device-to-device copies of n doubles (checkpoints, a tape's first velocity and scalars)
 __global__ void ak_copy_d(const double *__restrict__ src, double *__restrict__ dst, long long n) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    dst[i] = src[i];
-}
-__global__ void ak_copy_i(const int *__restrict__ src, int *__restrict__ dst, long long n) {
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
     dst[i] = src[i];
 }
