@@ -325,7 +325,10 @@ struct fsibe_adjoint {
   std::vector<SimSnap> snaps;
   AdjTape tape;
   double2 *lW = nullptr, *lNL = nullptr, *T[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-  double *lu1 = nullptr, *lu2 = nullptr, *lm = nullptr, *lvx = nullptr, *lvy = nullptr;
+  double *lu1 = nullptr, *lu2 = nullptr;
+  // the mask's adjoints of step j in [j & 1]: the row kernel adds to one
+  // step's while it assigns the step's before
+  double *lm[2] = {}, *lvx[2] = {}, *lvy[2] = {};
   double *part = nullptr, *h_part = nullptr;
   int part_blocks = 0;
   double *d_nodes = nullptr;
@@ -396,9 +399,8 @@ extern "C" int fsibe_adjoint_create_binomial(const fsibe_params *p, const double
   for (int k = 0; k < 6; ++k) a->T[k] = reinterpret_cast<double2 *>(D(sizeof(double2) * NH));
   a->lu1 = reinterpret_cast<double *>(D(sizeof(double) * N));
   a->lu2 = reinterpret_cast<double *>(D(sizeof(double) * N));
-  a->lm = reinterpret_cast<double *>(D(sizeof(double) * N));
-  a->lvx = reinterpret_cast<double *>(D(sizeof(double) * N));
-  a->lvy = reinterpret_cast<double *>(D(sizeof(double) * N));
+  for (int k = 0; k < 2; ++k)
+    for (double **q : {&a->lm[k], &a->lvx[k], &a->lvy[k]}) *q = reinterpret_cast<double *>(D(sizeof(double) * N));
   a->part_blocks = 256;
   a->part = reinterpret_cast<double *>(D(sizeof(double) * 4 * a->part_blocks * cap));
   a->d_nodes = reinterpret_cast<double *>(D(sizeof(double) * std::max(s->ns, 1)));
@@ -489,38 +491,141 @@ static void motion601_jac(const fsibe_params &p, double t, double jac[4][8]) {
   }
 }
 
-static int adj_reverse_step(fsibe_adjoint *a, int j, const double *u1n, double cJ) {
-  fsibe_sim *s = a->s;
-  AdjTape &t = a->tape;
+// fn(shape) for the fused row kernel / column kernel of the reverse sweep;
+// false if the grid has none (other lengths, and rows of more than 512
+// values, whose six buffers leave too few rows on a CU)
+template <class Fn>
+static bool with_adj_row(int H, Fn &&fn) {
+  switch (H) {
+    case 32: fn(AdjRowShape<32, 4>{}); return true;
+    case 48: fn(AdjRowShape<48, 8>{}); return true;
+    case 64: fn(AdjRowShape<64, 8>{}); return true;
+    case 96: fn(AdjRowShape<96, 16>{}); return true;
+    case 128: fn(AdjRowShape<128, 16>{}); return true;
+    case 192: fn(AdjRowShape<192, 32>{}); return true;
+    case 256: fn(AdjRowShape<256, 32>{}); return true;
+    default: return false;
+  }
+}
+template <class Fn>
+static bool with_adj_col(int ny, Fn &&fn) {
+  switch (ny) {
+    case 64: fn(AdjColShape<64, 8>{}); return true;
+    case 96: fn(AdjColShape<96, 12>{}); return true;
+    case 128: fn(AdjColShape<128, 16>{}); return true;
+    case 192: fn(AdjColShape<192, 24>{}); return true;
+    case 256: fn(AdjColShape<256, 32>{}); return true;
+    case 384: fn(AdjColShape<384, 48>{}); return true;
+    case 512: fn(AdjColShape<512, 64>{}); return true;
+    default: return false;
+  }
+}
+
+// a recorded step's mask box
+static MaskBox tape_box(const AdjTape &t, int j) {
   const AdjTape::Rec &r = t.rec[j];
   MaskBox mb;
   mb.x0 = r.mbox.x0; mb.x1 = r.mbox.x1; mb.y0 = r.mbox.y0; mb.y1 = r.mbox.y1; mb.w = r.mbox.w();
   if (r.mbox.empty()) { mb.x0 = 0; mb.x1 = -1; mb.y0 = 0; mb.y1 = -1; mb.w = 0; }
   mb.m = t.m + j * t.N; mb.vx = t.vx + j * t.N; mb.vy = t.vy + j * t.N;
+  return mb;
+}
+
+// rows: the nonlinear term's adjoint of step jn (< 0: none), then the
+// velocity's and J's of step jv (< 0: none); u1n is the velocity step jv ended
+// with, cJ its weight in J
+static int adj_rows(fsibe_adjoint *a, int jn, int jv, const double *u1n, double cJ) {
+  fsibe_sim *s = a->s;
+  AdjTape &t = a->tape;
   double2 *Ta = a->T[0], *Tb = a->T[1], *Tc = a->T[2], *Td = a->T[3], *Te = a->T[4], *Tf = a->T[5];
+  const double *ms = s->sponge_on ? s->ms : nullptr;
+  int rc = FSIBE_OK;
+  const bool fused = with_adj_row(s->H, [&](auto S) {
+    using ST = decltype(S);
+    AdjRowArgs r{};
+    r.lu1 = a->lu1; r.lu2 = a->lu2; r.c = s->sc;
+    if (jn >= 0) {
+      const int k = jn & 1;
+      r.Tc = Tc; r.Td = Td; r.A = t.A + jn * t.NH; r.B = t.B + jn * t.NH; r.u1 = t.u1 + jn * t.N;
+      r.u2 = t.u2 + jn * t.N; r.ms = ms; r.mb = tape_box(t, jn); r.penal_on = s->penal_on;
+      r.lm = a->lm[k]; r.lvx = a->lvx[k]; r.lvy = a->lvy[k]; r.Te = Te; r.Tf = Tf;
+    }
+    if (jv >= 0) {
+      const int k = jv & 1;
+      r.u1n = u1n; r.mbv = tape_box(t, jv); r.win = t.rec[jv].win; r.cJ = cJ;
+      r.lmv = a->lm[k]; r.lvxv = a->lvx[k]; r.lvyv = a->lvy[k]; r.Ta = Ta; r.Tb = Tb;
+    }
+    rc = [&]() -> int {
+      KLAUNCH(ak_row_step<ST>, s->ny, ST::THREADS, ST::LDS, s->stream, r, s->twx);
+      return FSIBE_OK;
+    }();
+  });
+  if (fused) return rc;
+  if (jn >= 0) {
+    const int k = jn & 1;
+    const MaskBox mb = tape_box(t, jn);
+    CHK(with_rows<6>(s->px, [&](auto F, int nt) -> int {
+      KLAUNCH(ak_rows_nl<decltype(F)>, s->ny, nt, sizeof(double2) * 6 * padlen(s->H), s->stream, Tc, Td,
+              t.A + jn * t.NH, t.B + jn * t.NH, t.u1 + jn * t.N, t.u2 + jn * t.N, ms, mb, (int)s->penal_on, a->lu1,
+              a->lu2, a->lm[k], a->lvx[k], a->lvy[k], Te, Tf, F, s->twx, s->sc);
+      return FSIBE_OK;
+    }));
+  }
+  if (jv >= 0) {
+    const int k = jv & 1;
+    const MaskBox mb = tape_box(t, jv);
+    CHK(with_rows<2>(s->px, [&](auto F, int nt) -> int {
+      KLAUNCH(ak_rows_vel<decltype(F)>, s->ny, nt, sizeof(double2) * 2 * padlen(s->H), s->stream, a->lu1, a->lu2,
+              u1n, mb, t.rec[jv].win, cJ, a->lm[k], a->lvx[k], a->lvy[k], Ta, Tb, F, s->twx, s->sc);
+      return FSIBE_OK;
+    }));
+  }
+  return FSIBE_OK;
+}
+
+// columns: K1's adjoint of step jn (< 0: none), then the update's of step jv
+// (< 0: none)
+static int adj_cols(fsibe_adjoint *a, int jn, int jv) {
+  fsibe_sim *s = a->s;
+  AdjTape &t = a->tape;
+  double2 *Ta = a->T[0], *Tb = a->T[1], *Tc = a->T[2], *Td = a->T[3], *Te = a->T[4], *Tf = a->T[5];
+  int rc = FSIBE_OK;
+  const bool fused = with_adj_col(s->ny, [&](auto S) {
+    using ST = decltype(S);
+    AdjColArgs r{};
+    r.lW = a->lW; r.lNL = a->lNL; r.c = s->sc;
+    if (jn >= 0) { r.Te = Te; r.Tf = Tf; }
+    if (jv >= 0) {
+      r.Ta = Ta; r.Tb = Tb; r.Tc = Tc; r.Td = Td; r.s = t.sc + jv;
+      r.explicit_step = t.rec[jv].explicit_step;
+    }
+    rc = [&]() -> int {
+      KLAUNCH(ak_col_step<ST>, s->H, ST::THREADS, ST::LDS, s->stream, r, s->twy);
+      return FSIBE_OK;
+    }();
+  });
+  if (fused) return rc;
+  if (jn >= 0)
+    CHK(with_cols<2>(s->py, s->H, pick_tx(s->H, s->ny, 2, 1), [&](auto F, int nt, int TX) -> int {
+      KLAUNCH(ak_cols_w0<decltype(F)>, s->H / TX, nt, sizeof(double2) * 2 * TX * padlen(s->ny), s->stream, Te, Tf,
+              a->lW, F, s->twy, s->sc);
+      return FSIBE_OK;
+    }));
+  if (jv >= 0)
+    CHK(with_cols<2>(s->py, s->H, pick_tx(s->H, s->ny, 2, 1), [&](auto F, int nt, int TX) -> int {
+      KLAUNCH(ak_cols_ab2<decltype(F)>, s->H / TX, nt, sizeof(double2) * 2 * TX * padlen(s->ny), s->stream, Ta, Tb,
+              a->lW, a->lNL, Tc, Td, t.sc + jv, t.rec[jv].explicit_step, F, s->twy, s->sc);
+      return FSIBE_OK;
+    }));
+  return FSIBE_OK;
+}
+
+// the motion parameters' partial sums of step j
+static int adj_mask_part(fsibe_adjoint *a, int j) {
+  fsibe_sim *s = a->s;
+  AdjTape &t = a->tape;
+  const AdjTape::Rec &r = t.rec[j];
   const size_t nbox = r.mbox.empty() ? 0 : (size_t)r.mbox.w() * r.mbox.h();
-  CHK(with_rows<2>(s->px, [&](auto F, int nt) -> int {
-    KLAUNCH(ak_rows_vel<decltype(F)>, s->ny, nt, sizeof(double2) * 2 * padlen(s->H), s->stream, a->lu1, a->lu2,
-            u1n, mb, r.win, cJ, a->lm, a->lvx, a->lvy, Ta, Tb, F, s->twx, s->sc);
-    return FSIBE_OK;
-  }));
-  CHK(with_cols<2>(s->py, s->H, pick_tx(s->H, s->ny, 2, 1), [&](auto F, int nt, int TX) -> int {
-    KLAUNCH(ak_cols_ab2<decltype(F)>, s->H / TX, nt, sizeof(double2) * 2 * TX * padlen(s->ny), s->stream, Ta, Tb,
-            a->lW, a->lNL, Tc, Td, t.sc + j, r.explicit_step, F, s->twy, s->sc);
-    return FSIBE_OK;
-  }));
-  CHK(with_rows<6>(s->px, [&](auto F, int nt) -> int {
-    KLAUNCH(ak_rows_nl<decltype(F)>, s->ny, nt, sizeof(double2) * 6 * padlen(s->H), s->stream, Tc, Td,
-            t.A + j * t.NH, t.B + j * t.NH, t.u1 + j * t.N, t.u2 + j * t.N,
-            s->sponge_on ? s->ms : nullptr, mb, (int)s->penal_on, a->lu1, a->lu2, a->lm, a->lvx, a->lvy, Te, Tf,
-            F, s->twx, s->sc);
-    return FSIBE_OK;
-  }));
-  CHK(with_cols<2>(s->py, s->H, pick_tx(s->H, s->ny, 2, 1), [&](auto F, int nt, int TX) -> int {
-    KLAUNCH(ak_cols_w0<decltype(F)>, s->H / TX, nt, sizeof(double2) * 2 * TX * padlen(s->ny), s->stream, Te, Tf,
-            a->lW, F, s->twy, s->sc);
-    return FSIBE_OK;
-  }));
   double *part = a->part + (size_t)j * 4 * a->part_blocks;
   if (nbox > 0) {
     double alpha, at, att, LE[6];
@@ -532,7 +637,7 @@ static int adj_reverse_step(fsibe_adjoint *a, int j, const double *u1n, double c
     RigidBeam rb;
     rb.LEx = LE[0]; rb.LEy = LE[1]; rb.alpha = alpha; rb.hdot = LE[3]; rb.at = at;
     rb.s = a->d_nodes; rb.ns = s->ns; rb.off = s->p.iCylinder == 1 ? 1 : 0;
-    ak_mask<<<a->part_blocks, 256, 0, s->stream>>>(t.win + j * t.N, a->lm, a->lvx, a->lvy, mc, rb, r.mbox.x0,
+    ak_mask<<<a->part_blocks, 256, 0, s->stream>>>(t.win + j * t.N, a->lm[j & 1], a->lvx[j & 1], a->lvy[j & 1], mc, rb, r.mbox.x0,
                                                   r.mbox.y0, r.mbox.w(), r.mbox.h(), part);
     HIPCHK(hipGetLastError());
   } else {
@@ -582,9 +687,13 @@ static int adj_record_reverse(fsibe_adjoint *a, int k, double *J, double *T, dou
     *T = s->jsum_t;
   }
   const double dxdy = s->dx * s->dy;
-  for (int j = len - 1; j >= 0; --j) {
-    const double *u1n = j == len - 1 ? s->u1 : t.u1 + (size_t)(j + 1) * t.N;
-    CHK(adj_reverse_step(a, j, u1n, -(t.rec[j].dt1 * dxdy) / *T));
+  for (int j = len; j >= 0; --j) {
+    // rows and columns: step j's first halves with step j-1's second ones
+    const int jn = j < len ? j : -1, jv = j - 1;
+    const double *u1n = j == len ? s->u1 : t.u1 + (size_t)j * t.N;
+    CHK(adj_rows(a, jn, jv, u1n, jv >= 0 ? -(t.rec[jv].dt1 * dxdy) / *T : 0.0));
+    if (jn >= 0) CHK(adj_mask_part(a, jn));
+    CHK(adj_cols(a, jn, jv));
   }
   HIPCHK(hipMemcpyAsync(a->h_part, a->part, sizeof(double) * 4 * a->part_blocks * len, hipMemcpyDeviceToHost,
                         s->stream));

@@ -21,6 +21,7 @@
 //   row r2c (unnormalised) R             -> f = c2r(Y), Y0 = X0, Yk = Xk / 2
 //   spectral multiplier m                -> conj(m)
 #pragma once
+#include "kernels_fused.hpp"
 #include "kernels_mask.hpp"
 #include "kernels_step.hpp"
 
@@ -277,6 +278,311 @@ __global__ void __launch_bounds__(FY::LB) ak_cols_w0(const double2 *__restrict__
     const double2 l = lW[g];
     lW[g] = make_double2(l.x + (ye.x + kyf * yf.y), l.y + (ye.y - kyf * yf.x));
   }
+}
+
+// ---- the reverse step in two kernels ----------------------------------------
+// Where the grid has the shapes: one row kernel takes ak_rows_nl of step j
+// and ak_rows_vel of step j-1 (dJ/du passes in registers and LDS), one column
+// kernel ak_cols_w0 of step j and ak_cols_ab2 of step j-1 (lW is read and
+// written once).  Either half may be absent: the last step of a unit starts
+// with the second halves alone, the first one ends with the first halves.
+// Both are bound by the latency of their chains of transforms at 512^2: the
+// four kernels took 12.8 + 8.5 and 6.9 + 14.0 us there, these two 16.9 and 12.8.
+struct AdjRowArgs {
+  // ak_rows_nl (Te null: absent)
+  const double2 *Tc, *Td, *A, *B;
+  const double *u1, *u2, *ms;
+  MaskBox mb;
+  int penal_on;
+  double *lm, *lvx, *lvy;
+  double2 *Te, *Tf;
+  // dJ/du: written by the first half without the second, read by the second
+  // without the first
+  double *lu1, *lu2;
+  // ak_rows_vel (Ta null: absent)
+  const double *u1n;
+  MaskBox mbv;
+  Window win;
+  double cJ;
+  double *lmv, *lvxv, *lvyv;
+  double2 *Ta, *Tb;
+  StepConsts c;
+};
+
+// one row by six slots of NT threads: the six inverse transforms, then the
+// forward ones of dJ/du (slots 0, 1) and of l(omega), l(omega_y), l(omega_x)
+template <int H, int NT>
+__device__ __forceinline__ void adj_row_body(const AdjRowArgs &a, const double2 *__restrict__ twx, int y) {
+#pragma clang fp contract(off)
+  extern __shared__ double2 lds[];
+  constexpr int PL = padlen(H), nx = 2 * H, NR = 6 * NT, PN = (H + NR - 1) / NR;
+  constexpr bool WAVE = NR <= 64;
+  using Out = FftOut<H, NT>;
+  const int p = threadIdx.x, slot = p / NT, t = p - slot * NT;
+  double2 *xb = lds + slot * PL;
+  const size_t rowk = (size_t)y * H, rowx = (size_t)y * nx;
+  const double sx = a.c.sx;
+  const bool nl = a.Te != nullptr, vel = a.Ta != nullptr;
+  FftTw<H, NT> T;
+  T.load(twx, 2, t);
+  double2 z[Out::N];
+  auto put = [&]() {
+#pragma unroll
+    for (int i = 0; i < Out::ITEMS; ++i) {
+      if (Out::M % NT != 0 && t + i * NT >= Out::M) continue;
+#pragma unroll
+      for (int r = 0; r < Out::R; ++r) xb[pidx(t + i * NT + r * Out::M)] = z[i * Out::R + r];
+    }
+  };
+  if (nl) {
+    const double2 *pA = a.A, *pB = a.B, *pC = a.Tc, *pD = a.Td;
+    const double2 *src = (slot == 0 || slot == 2 ? pA : slot == 1 ? pB : slot == 5 ? pD : pC) + rowk;
+    auto at = [&](int k) {
+      const double2 v = src[k];
+      const double kf = (double)k * sx;
+      if (slot < 2) return v;
+      if (slot == 2) return make_double2(-kf * v.y, kf * v.x);
+      // transposes of the unnormalised r2c: Y0 = X0, Yk = Xk / 2 (k >= 1)
+      const double hk = k == 0 ? 1.0 : 0.5;
+      if (slot == 4) return make_double2(hk * (kf * v.y), hk * (-(kf * v.x)));
+      return make_double2(hk * v.x, hk * v.y);
+    };
+    fft_io<H, NT, true, 1, WAVE, false>(
+        xb, T, t, true,
+        [&](int, int, int e) { return c2r_elem(at(e), at(e == 0 ? 0 : H - e), e, cconj(twx[e])); },
+        [&](int i, int r, int, double2 x) { z[i * Out::R + r] = x; });
+    grp_sync<WAVE>();
+    put();
+    grp_sync<WAVE>();
+  }
+  const MaskBox mb = a.mb, mbv = a.mbv;
+  const bool prow = nl && a.penal_on && mb.x1 >= mb.x0 && y >= mb.y0 && y <= mb.y1;
+  const bool mrow = vel && mbv.x1 >= mbv.x0 && y >= mbv.y0 && y <= mbv.y1;
+  const bool wrow = y >= a.win.y0 && y <= a.win.y1;
+#pragma unroll
+  for (int k = 0; k < PN; ++k) {
+    const int n = p + k * NR;
+    if (H % NR != 0 && n >= H) continue;
+    const int q = pidx(n);
+    double2 lu1v, lu2v;
+    if (nl) {
+      const double2 w = lds[q], wy = lds[PL + q], wx = lds[2 * PL + q];
+      const double2 lr = lds[3 * PL + q], lpy = lds[4 * PL + q], lpx = lds[5 * PL + q];
+      const double2 a1 = reinterpret_cast<const double2 *>(a.u1 + rowx)[n];
+      const double2 a2 = reinterpret_cast<const double2 *>(a.u2 + rowx)[n];
+      double2 s = make_double2(0.0, 0.0);
+      if (a.ms) s = reinterpret_cast<const double2 *>(a.ms + rowx)[n];
+      (void)w;
+      // r = -u1 wx - u2 wy - s w
+      lu1v = make_double2(-(wx.x * lr.x), -(wx.y * lr.y));
+      lu2v = make_double2(-(wy.x * lr.x), -(wy.y * lr.y));
+      if (prow) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int x = 2 * n + h;
+          if (!mb.inside(x, y)) continue;
+          const size_t qq = (size_t)(y - mb.y0) * mb.w + (x - mb.x0);
+          const double m = mb.m[qq], vx = mb.vx[qq], vy = mb.vy[qq];
+          const double uu1 = h ? a1.y : a1.x, uu2 = h ? a2.y : a2.x;
+          const double gpx = h ? lpx.y : lpx.x, gpy = h ? lpy.y : lpy.x;
+          // px = -m (u1 - vx), py = -m (u2 - vy)
+          if (h) { lu1v.y += -(m * gpx); lu2v.y += -(m * gpy); }
+          else { lu1v.x += -(m * gpx); lu2v.x += -(m * gpy); }
+          a.lvx[qq] += m * gpx;
+          a.lvy[qq] += m * gpy;
+          a.lm[qq] += -((uu1 - vx) * gpx) - (uu2 - vy) * gpy;
+        }
+      }
+      lds[3 * PL + q] = make_double2(-(s.x * lr.x), -(s.y * lr.y));
+      lds[4 * PL + q] = make_double2(-(a2.x * lr.x), -(a2.y * lr.y));
+      lds[5 * PL + q] = make_double2(-(a1.x * lr.x), -(a1.y * lr.y));
+      if (!vel) {
+        reinterpret_cast<double2 *>(a.lu1 + rowx)[n] = lu1v;
+        reinterpret_cast<double2 *>(a.lu2 + rowx)[n] = lu2v;
+      }
+    } else {
+      lu1v = reinterpret_cast<const double2 *>(a.lu1 + rowx)[n];
+      lu2v = reinterpret_cast<const double2 *>(a.lu2 + rowx)[n];
+    }
+    if (vel) {
+      if (mrow) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int x = 2 * n + h;
+          if (!mbv.inside(x, y)) continue;
+          const size_t qq = (size_t)(y - mbv.y0) * mbv.w + (x - mbv.x0);
+          double gm = 0.0, gvx = 0.0;
+          if (wrow && x >= a.win.x0 && x <= a.win.x1) {
+            const double m = mbv.m[qq], uu = a.u1n[rowx + x];
+            gm = a.cJ * (uu - mbv.vx[qq]);
+            gvx = -(a.cJ * m);
+            if (h) lu1v.y += a.cJ * m; else lu1v.x += a.cJ * m;
+          }
+          a.lmv[qq] = gm;
+          a.lvxv[qq] = gvx;
+          a.lvyv[qq] = 0.0;
+        }
+      }
+      lds[q] = lu1v;
+      lds[PL + q] = lu2v;
+    }
+  }
+  grp_sync<WAVE>();
+  const bool act = slot < 2 ? vel : slot > 2 && nl;
+  fft_io<H, NT, false, 1, WAVE, false>(
+      xb, T, t, act, [&](int, int, int e) { return xb[pidx(e)]; },
+      [&](int i, int r, int, double2 x) { z[i * Out::R + r] = x; });
+  grp_sync<WAVE>();
+  if (act) put();
+  grp_sync<WAVE>();
+#pragma unroll
+  for (int i = 0; i < PN; ++i) {
+    const int k = p + i * NR;
+    if (H % NR != 0 && k >= H) continue;
+    const int q = pidx(k), qm = pidx(k == 0 ? 0 : H - k);
+    const double wk = k == 0 ? 1.0 : 2.0, kf = (double)k * sx;
+    const double2 tw = twx[k];
+    if (vel) {
+      const double2 xa = r2c_one(lds[q], lds[qm], tw), xb2 = r2c_one(lds[PL + q], lds[PL + qm], tw);
+      a.Ta[rowk + k] = make_double2(wk * xa.x, wk * xa.y);
+      // i kx (wk xb)
+      a.Tb[rowk + k] = make_double2(-(kf * (wk * xb2.y)), kf * (wk * xb2.x));
+    }
+    if (nl) {
+      const double2 xw = r2c_one(lds[3 * PL + q], lds[3 * PL + qm], tw);
+      const double2 xwy = r2c_one(lds[4 * PL + q], lds[4 * PL + qm], tw);
+      const double2 xwx = r2c_one(lds[5 * PL + q], lds[5 * PL + qm], tw);
+      // dA = R^T l(w) + conj(i kx) R^T l(wx), dB = R^T l(wy)
+      a.Te[rowk + k] = make_double2(wk * (xw.x + kf * xwx.y), wk * (xw.y - kf * xwx.x));
+      a.Tf[rowk + k] = make_double2(wk * xwy.x, wk * xwy.y);
+    }
+  }
+}
+template <int HC, int NTC> struct AdjRowShape {
+  static constexpr int H = HC, NT = NTC, THREADS = 6 * NTC;
+  static constexpr size_t LDS = sizeof(double2) * 6 * padlen(H);
+};
+template <class S>
+__global__ void __launch_bounds__(S::THREADS) ak_row_step(AdjRowArgs a, const double2 *__restrict__ twx) {
+  adj_row_body<S::H, S::NT>(a, twx, blockIdx.x);
+}
+
+struct AdjColArgs {
+  const double2 *Te, *Tf;  // ak_cols_w0 (Te null: absent)
+  const double2 *Ta, *Tb;  // ak_cols_ab2 (Ta null: absent)
+  double2 *lW, *lNL, *Tc, *Td;
+  const DevScalars *s;
+  int explicit_step;
+  StepConsts c;
+};
+
+// one column by four slots of NT threads: the four forward transforms, the
+// spectral transposes, two inverse transforms
+template <int L, int NT>
+__device__ __forceinline__ void adj_col_body(const AdjColArgs &a, const double2 *__restrict__ twy, int bid, int nblk) {
+#pragma clang fp contract(off)
+  extern __shared__ double2 lds[];
+  constexpr int PL = padlen(L), NTHR = 4 * NT, EL = (L + NTHR - 1) / NTHR;
+  constexpr bool WAVE = NTHR <= 64;
+  using Out = FftOut<L, NT>;
+  const StepConsts &c = a.c;
+  const int tid = threadIdx.x, H = c.H, slot = tid / NT, t = tid - slot * NT;
+  const int kx = xcd_remap(bid, nblk);
+  double2 *xb = lds + slot * PL;
+  const bool w0 = a.Te != nullptr, ab2 = a.Ta != nullptr;
+  FftTw<L, NT> T;
+  T.load(twy, 1, t);
+  double cx1 = 0.0, cy1 = 0.0, cx0 = 0.0, cy0 = 0.0, b10 = 0.0, b11 = 0.0;
+  if (ab2) { cx1 = a.s->cx1; cy1 = a.s->cy1; cx0 = a.s->cx0; cy0 = a.s->cy0; b10 = a.s->b10; b11 = a.s->b11; }
+  double2 lw[EL], ln[EL];
+#pragma unroll
+  for (int q = 0; q < EL; ++q) {
+    const int idx = tid + q * NTHR;
+    lw[q] = ln[q] = make_double2(0.0, 0.0);
+    if (L % NTHR == 0 || idx < L) {
+      lw[q] = a.lW[(size_t)idx * H + kx];
+      if (ab2) ln[q] = a.lNL[(size_t)idx * H + kx];
+    }
+  }
+  {
+    double2 z[Out::N];
+    const double2 *pe = a.Te, *pf = a.Tf, *pa = a.Ta, *pb = a.Tb;
+    const double2 *src = slot == 0 ? pe : slot == 1 ? pf : slot == 2 ? pa : pb;
+    const bool act = src != nullptr;
+    fft_io<L, NT, false, 1, WAVE, false>(
+        xb, T, t, act, [&](int, int, int e) { return src[(size_t)e * H + kx]; },
+        [&](int i, int r, int, double2 x) { z[i * Out::R + r] = x; });
+    grp_sync<WAVE>();
+    if (act) {
+#pragma unroll
+      for (int i = 0; i < Out::ITEMS; ++i) {
+        if (Out::M % NT != 0 && t + i * NT >= Out::M) continue;
+#pragma unroll
+        for (int r = 0; r < Out::R; ++r) xb[pidx(t + i * NT + r * Out::M)] = z[i * Out::R + r];
+      }
+    }
+    grp_sync<WAVE>();
+  }
+  const bool same = cx0 == cx1 && cy0 == cy1;
+  const double rx = 1.0 / c.kxt2, ry = 1.0 / c.kyt2, kx2 = (double)(kx * kx);
+#pragma unroll
+  for (int q = 0; q < EL; ++q) {
+    const int idx = tid + q * NTHR;
+    if (L % NTHR != 0 && idx >= L) continue;
+    const size_t g = (size_t)idx * H + kx;
+    const int ky = ky_signed(idx, L), aky = ky < 0 ? -ky : ky;
+    const double kyf = (double)ky * c.sy, ky2 = (double)(aky * aky);
+    double2 *l0 = lds + pidx(idx);
+    double2 l = lw[q];
+    if (w0) {
+      const double2 ye = l0[0], yf = l0[PL];
+      l = idx == L / 2 ? make_double2(0.0, 0.0)
+                       : make_double2(l.x + (ye.x + kyf * yf.y), l.y + (ye.y - kyf * yf.x));
+    }
+    if (!ab2) {
+      a.lW[g] = l;
+      continue;
+    }
+    double2 lnl = make_double2(0.0, 0.0), lw0 = lnl, lnl1 = lnl;
+    if (idx != L / 2) {
+      const double2 ya = l0[2 * PL], yb = l0[3 * PL];
+      // d psi = -i ky Ya + Yb, then the Poisson factor (psi = W1 / |k|^2)
+      const double2 lpsi = make_double2(kyf * ya.y + yb.x, -(kyf * ya.x) + yb.y);
+      if (!(kx == 0 && ky == 0)) {
+        const double quot = (kx2 * c.scalex + ky2 * c.scaley), rq = 1.0 / quot;
+        l.x += div_by(lpsi.x, quot, rq);
+        l.y += div_by(lpsi.y, quot, rq);
+      }
+      const double v1 = exp(cx1 * kx2 + cy1 * ky2);
+      const double f = v1 * dealias_fast(c, kx, aky, rx, ry);
+      lw0 = make_double2(f * l.x, f * l.y);
+      lnl = make_double2(b10 * lw0.x + ln[q].x, b10 * lw0.y + ln[q].y);
+      if (!a.explicit_step) {
+        const double v0 = same ? v1 : exp(cx0 * kx2 + cy0 * ky2);
+        lnl1 = make_double2(b11 * v0 * lw0.x, b11 * v0 * lw0.y);
+      }
+    }
+    a.lW[g] = lw0;
+    a.lNL[g] = lnl1;
+    // nl = norm Cfwd(Rc) - i ky norm Cfwd(Rpx):  dRc = norm Cinv(lnl), dRpx = norm Cinv(i ky lnl)
+    l0[0] = make_double2(c.norm * lnl.x, c.norm * lnl.y);
+    l0[PL] = make_double2(c.norm * (-(kyf * lnl.y)), c.norm * (kyf * lnl.x));
+  }
+  if (!ab2) return;
+  grp_sync<WAVE>();
+  double2 *oc = a.Tc, *od = a.Td;
+  double2 *out = slot == 0 ? oc : od;
+  fft_io<L, NT, true, 1, WAVE, false>(
+      xb, T, t, slot < 2, [&](int, int, int e) { return xb[pidx(e)]; },
+      [&](int, int, int e, double2 x) { out[(size_t)e * H + kx] = x; });
+}
+template <int LC, int NTC> struct AdjColShape {
+  static constexpr int L = LC, NT = NTC, THREADS = 4 * NTC;
+  static constexpr size_t LDS = sizeof(double2) * 4 * padlen(L);
+};
+template <class S>
+__global__ void __launch_bounds__(S::THREADS) ak_col_step(AdjColArgs a, const double2 *__restrict__ twy) {
+  adj_col_body<S::L, S::NT>(a, twy, blockIdx.x, gridDim.x);
 }
 
 // ---- ak_mask: d(mask)/d(kinematics) of a rigid beam -------------------------

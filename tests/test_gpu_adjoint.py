@@ -192,3 +192,31 @@ def test_unsupported_configurations_are_refused():
     for kw in (dict(iFLUSI=1), dict(iMotion=600), dict(iSharpTrailing=1), dict(dt_fixed=0.0)):
         with pytest.raises(FsibeError):
             Adjoint(Params(nx=64, ny=64, ns=24, **({"iMotion": 601} | kw)), None, 10, 5)
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 96), (96, 64), (128, 192), (192, 128), (384, 256), (256, 384), (72, 64),
+                                   (64, 72), (108, 108)])
+def test_directional_derivative_on_every_form_of_the_reverse_step(nx, ny):
+    """the reverse sweep's fused row and column kernels, each with and without
+    its halves (units of 5 and 2 steps), on lengths that have both, one or
+    none: the gradient along a direction against the central difference of
+    J along it, as on the workload"""
+    from fsibe_2d_amd import Params
+    from fsibe_2d_amd.adjoint import Adjoint
+    from fsibe_2d_amd.inputs import half_to_packed, normals
+
+    p = Params(nx=nx, ny=ny, ns=33, nu=2e-3, dt_fixed=2e-4, cfl=100.0, iMotion=601,
+               heave_freq=2.0, iSaveBeam=0, iSmoothCutoff=1)
+    z = np.zeros((ny, nx // 2), dtype=np.complex128)
+    q = np.array(normals(5, 2 * 6 * 7)).reshape(2, 6, 7)
+    z[1:7, 1:7] = (1e-3 * (q[0] + 1j * q[1]))[:, 1:]
+    c = _coef()
+    d = np.array(normals(4, 8))
+    d /= np.linalg.norm(d)
+    a = Adjoint(p, half_to_packed(z), 12, 5)
+    J, g = a.gradient(c)
+    h = 1e-6
+    fd = (a.objective(c + h * d) - a.objective(c - h * d)) / (2 * h)
+    print(f"[adjoint {nx}x{ny}] J {J:.10e} g.d {g @ d:.10e} fd {fd:.10e}", flush=True)
+    assert abs(g @ d - fd) <= 1e-6 * abs(fd)
+    a.close()
