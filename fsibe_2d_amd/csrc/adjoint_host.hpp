@@ -50,6 +50,7 @@ struct AdjTape {
     Window win;
     double tau = 0.0, dt1 = 0.0;
     int explicit_step = 0;
+    int kc = 0;  // columns of A, B in use
   };
   std::vector<Rec> rec;
 };
@@ -120,6 +121,7 @@ static int tape_fluid(fsibe_sim *s, bool explicit_step) {
   s->u1 = more ? t.u1 + (j + 1) * t.N : t.own.u1;
   s->u2 = more ? t.u2 + (j + 1) * t.N : t.own.u2;
   t.rec[j].explicit_step = explicit_step ? 1 : 0;
+  t.rec[j].kc = s->kcA;
   t.n = (int)j + 1;
   return FSIBE_OK;
 }
@@ -521,6 +523,11 @@ static bool with_adj_col(int ny, Fn &&fn) {
   }
 }
 
+// columns of the adjoint fields in use, in whole groups of 8 (xcd_remap)
+static int adj_kl(const fsibe_sim *s) {
+  return with_adj_row(s->H, [](auto) {}) && with_adj_col(s->ny, [](auto) {}) ? std::min(s->H, (s->sc.kc + 7) & ~7) : s->H;
+}
+
 // a recorded step's mask box
 static MaskBox tape_box(const AdjTape &t, int j) {
   const AdjTape::Rec &r = t.rec[j];
@@ -543,9 +550,10 @@ static int adj_rows(fsibe_adjoint *a, int jn, int jv, const double *u1n, double 
   const bool fused = with_adj_row(s->H, [&](auto S) {
     using ST = decltype(S);
     AdjRowArgs r{};
-    r.lu1 = a->lu1; r.lu2 = a->lu2; r.c = s->sc;
+    r.lu1 = a->lu1; r.lu2 = a->lu2; r.c = s->sc; r.kl = adj_kl(s);
     if (jn >= 0) {
       const int k = jn & 1;
+      r.c.kc = t.rec[jn].kc;
       r.Tc = Tc; r.Td = Td; r.A = t.A + jn * t.NH; r.B = t.B + jn * t.NH; r.u1 = t.u1 + jn * t.N;
       r.u2 = t.u2 + jn * t.N; r.ms = ms; r.mb = tape_box(t, jn); r.penal_on = s->penal_on;
       r.lm = a->lm[k]; r.lvx = a->lvx[k]; r.lvy = a->lvy[k]; r.Te = Te; r.Tf = Tf;
@@ -564,10 +572,12 @@ static int adj_rows(fsibe_adjoint *a, int jn, int jv, const double *u1n, double 
   if (jn >= 0) {
     const int k = jn & 1;
     const MaskBox mb = tape_box(t, jn);
+    StepConsts c = s->sc;
+    c.kc = t.rec[jn].kc;
     CHK(with_rows<6>(s->px, [&](auto F, int nt) -> int {
       KLAUNCH(ak_rows_nl<decltype(F)>, s->ny, nt, sizeof(double2) * 6 * padlen(s->H), s->stream, Tc, Td,
               t.A + jn * t.NH, t.B + jn * t.NH, t.u1 + jn * t.N, t.u2 + jn * t.N, ms, mb, (int)s->penal_on, a->lu1,
-              a->lu2, a->lm[k], a->lvx[k], a->lvy[k], Te, Tf, F, s->twx, s->sc);
+              a->lu2, a->lm[k], a->lvx[k], a->lvy[k], Te, Tf, F, s->twx, c);
       return FSIBE_OK;
     }));
   }
@@ -600,7 +610,7 @@ static int adj_cols(fsibe_adjoint *a, int jn, int jv) {
       r.explicit_step = t.rec[jv].explicit_step;
     }
     rc = [&]() -> int {
-      KLAUNCH(ak_col_step<ST>, s->H, ST::THREADS, ST::LDS, s->stream, r, s->twy);
+      KLAUNCH(ak_col_step<ST>, adj_kl(s), ST::THREADS, ST::LDS, s->stream, r, s->twy);
       return FSIBE_OK;
     }();
   });

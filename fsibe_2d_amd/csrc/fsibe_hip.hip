@@ -1079,6 +1079,7 @@ struct fsibe_sim {
   // launch, or the previous step's fused row stage), into Rcp (T[2] or T[8])
   bool k2_ready = false;
   double2 *Bp = nullptr, *Rcp = nullptr;
+  int kcA = 0;  // the columns of both beyond are zero and not stored
   // launch choices of the column stages K1, K4, K5, K7 (the autotuner's,
   // once fsibe_run has measured them for this grid; else the static ones)
   ColSel csel[4];
@@ -1542,8 +1543,11 @@ extern "C" int fsibe_sim_create(const fsibe_params *pp, fsibe_sim **out) {
   {
     const double kxt = 2.0 / 3.0 * (double)(s->nx / 2 - 1), kyt = 2.0 / 3.0 * (double)(s->ny / 2 - 1);
     c.kxt2 = kxt * kxt; c.kyt2 = kyt * kyt;
+    c.rkxt2 = 1.0 / c.kxt2; c.rkyt2 = 1.0 / c.kyt2;
   }
   c.idealis = p.idealis == 1;
+  c.kc = s->H;
+  for (int k = s->H - 1; k >= 0 && c.idealis && s->H > kCutH && (double)k * (double)k / c.kxt2 + 0.0 / c.kyt2 >= 1.0; --k) c.kc = k;
   c.nu = p.nu; c.eps = p.eps; c.dx = s->dx; c.dy = s->dy;
   FlowParams &f = s->fp;
   f.iMeanVelocity = p.iMeanVelocity; f.penal_on = p.iBeam > 0 || p.iWalls > 0 || p.iCylinder > 0;
@@ -2184,12 +2188,14 @@ static int velocity_only(fsibe_sim *s, double time) {
   }
   const double UMx = s->p.U_mean_true * mx, UMy = s->p.U_mean_true * my;
   MaskBox mb = mask_box(s);
+  StepConsts c = s->sc;
+  c.kc = s->H;  // a spectrum that no update has dealiased
   return with_rows<3>(s->px, [&](auto F, int nt) -> int {
     KLAUNCH(k_rows_press<decltype(F)>, s->ny, nt, lds, s->stream, nullptr, s->T[1], s->T[2], s->u1, s->u2,
             s->vor_mean, mb, s->win[0], s->win[1], rows_dev(s, s->slot), s->umax_part, s->T[4], s->T[5], s->dscal, UMx,
             UMy, 0, 0,
             F, s->twx,
-            s->sc);
+            c);
     return FSIBE_OK;
   });
 }
@@ -2207,7 +2213,15 @@ static int launch_k1(fsibe_sim *s, int level, bool have_a = false) {
   CHK(cols_inv_fields(s, s->W[level], outs + f0, fsel + f0, (sp10 ? 3 : 2) - f0));
   prof_end(s, P_COLS_W0);
   s->Bp = s->T[1];
+  s->kcA = have_a ? s->sc.kc : s->H;
   return FSIBE_OK;
+}
+
+// the constants of K2: columns of A, B beyond kcA are zero and not stored
+static StepConsts nl_consts(const fsibe_sim *s) {
+  StepConsts c = s->sc;
+  c.kc = s->kcA;
+  return c;
 }
 
 // K2 of the next step without the penalisation term, on every row: it reads
@@ -2226,7 +2240,7 @@ static int launch_k2_ahead(fsibe_sim *s) {
   CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
     KLAUNCH(k_rows_nl<decltype(F)>, na + nb, nt, lds, s->stream, s->T[0], s->Bp, s->u1, s->u2,
             s->sponge_on ? s->ms : nullptr, none, (int)s->penal_on, s->T[2], s->penal_on ? s->T[3] : nullptr,
-            F, s->twx, s->sc,
+            F, s->twx, nl_consts(s),
             s->umax_part, s->ny, s->dscal, s->fp, 0.0, 0.0, 0, res_dev(s, s->slot), 0, na, b1 + 1, 0,
             s->penal_on ? s->rowpen : nullptr, (int)(s->p.iSponge == 10));
     return FSIBE_OK;
@@ -2314,7 +2328,7 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
       CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
         KLAUNCH_EV(k_rows_nl<decltype(F)>, s->ny, nt, lds, s->stream, s->ev_dt, s->T[0], s->Bp, s->u1, s->u2,
                    s->sponge_on ? s->ms : nullptr, mb, (int)s->penal_on, s->T[2], s->penal_on ? s->T[3] : nullptr,
-                   F, s->twx, s->sc,
+                   F, s->twx, nl_consts(s),
                    s->umax_part, s->ny, s->dscal, s->fp, time, dt0, (int)explicit_step, res_dev(s, s->slot), 0,
                    s->ny, 0, 1, s->penal_on ? s->rowpen : nullptr, (int)(s->p.iSponge == 10));
         return FSIBE_OK;
@@ -2323,7 +2337,7 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
       CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
         KLAUNCH(k_rows_nl<decltype(F)>, s->ny, nt, lds, s->stream, s->T[0], s->Bp, s->u1, s->u2,
                 s->sponge_on ? s->ms : nullptr, mb, (int)s->penal_on, s->T[2], s->penal_on ? s->T[3] : nullptr,
-                F, s->twx, s->sc,
+                F, s->twx, nl_consts(s),
                 s->umax_part, s->ny, s->dscal, s->fp, time, dt0, (int)explicit_step, res_dev(s, s->slot), 0, s->ny,
                 0, 1, s->penal_on ? s->rowpen : nullptr, (int)(s->p.iSponge == 10));
         return FSIBE_OK;
@@ -2424,6 +2438,7 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
     s->k1_ready = true;
     s->k1_level = n1;
     s->Bp = s->T[7];
+    s->kcA = s->sc.kc;
     if (conv) {
       s->k2_ready = true;
       s->Rcp = s->T[8];
@@ -3560,7 +3575,7 @@ static void fill_batch_args(fsibe_batch *b, BatchGroup &g, int j, fsibe_sim *s, 
     RowsNlArgs &a = reinterpret_cast<RowsNlArgs *>(A + g.off[B_K2])[j];
     a.A = s->T[0]; a.B = s->T[1]; a.u1 = s->u1; a.u2 = s->u2; a.ms = s->sponge_on ? s->ms : nullptr;
     a.mb = mb; a.penal_on = s->penal_on; a.nparts = s->ny; a.explicit_step = 0; a.nblk = s->ny;
-    a.Rc = s->T[2]; a.Rpx = s->T[3]; a.c = s->sc; a.umax_part = s->umax_part; a.sc = s->dscal; a.fl = s->fp;
+    a.Rc = s->T[2]; a.Rpx = s->T[3]; a.c = s->sc; a.c.kc = s->H; a.umax_part = s->umax_part; a.sc = s->dscal; a.fl = s->fp;
     a.time = s->time; a.dt0 = s->dt0; a.res = res_dev(s, s->slot);
     a.rpx_zero = s->p.iSponge == 10 ? 1 : 0;
     maxblk[B_K2] = std::max(maxblk[B_K2], a.nblk);

@@ -178,11 +178,11 @@ __global__ void __launch_bounds__(FX::LB) ak_rows_nl(const double2 *__restrict__
   double2 *f0 = lds, *f1 = lds + PL, *f2 = lds + 2 * PL;
   double2 *g0 = lds + 3 * PL, *g1 = lds + 4 * PL, *g2 = lds + 5 * PL;
   for (int k = tid; k < H; k += nt) {
-    const double2 a = A[(size_t)y * H + k];
+    const double2 a = live(A + (size_t)y * H, k, H, c.kc);
     const double kf = (double)k * c.sx;
     const int q = pidx(k);
     f0[q] = a;
-    f1[q] = B[(size_t)y * H + k];
+    f1[q] = live(B + (size_t)y * H, k, H, c.kc);
     f2[q] = make_double2(-kf * a.y, kf * a.x);
     // transposes of the unnormalised r2c: Y0 = X0, Yk = Xk / 2 (k >= 1)
     const double hk = k == 0 ? 1.0 : 0.5;
@@ -306,7 +306,11 @@ struct AdjRowArgs {
   double cJ;
   double *lmv, *lvxv, *lvyv;
   double2 *Ta, *Tb;
-  StepConsts c;
+  // columns of the adjoint fields in use: dJ/d vortk of a mode that dealiasing
+  // removes is multiplied by zero in the update before, so none is formed
+  // for the columns beyond (H where one of the two kernels is not the fused one)
+  int kl;
+  StepConsts c;  // kc: of A, B
 };
 
 // one row by six slots of NT threads: the six inverse transforms, then the
@@ -337,8 +341,9 @@ __device__ __forceinline__ void adj_row_body(const AdjRowArgs &a, const double2 
   if (nl) {
     const double2 *pA = a.A, *pB = a.B, *pC = a.Tc, *pD = a.Td;
     const double2 *src = (slot == 0 || slot == 2 ? pA : slot == 1 ? pB : slot == 5 ? pD : pC) + rowk;
+    const int kc = slot < 3 ? a.c.kc : a.kl;
     auto at = [&](int k) {
-      const double2 v = src[k];
+      const double2 v = live(src, k, H, kc);
       const double kf = (double)k * sx;
       if (slot < 2) return v;
       if (slot == 2) return make_double2(-kf * v.y, kf * v.x);
@@ -438,7 +443,7 @@ __device__ __forceinline__ void adj_row_body(const AdjRowArgs &a, const double2 
 #pragma unroll
   for (int i = 0; i < PN; ++i) {
     const int k = p + i * NR;
-    if (H % NR != 0 && k >= H) continue;
+    if ((H % NR != 0 && k >= H) || k >= a.kl) continue;
     const int q = pidx(k), qm = pidx(k == 0 ? 0 : H - k);
     const double wk = k == 0 ? 1.0 : 2.0, kf = (double)k * sx;
     const double2 tw = twx[k];
@@ -476,7 +481,7 @@ struct AdjColArgs {
   StepConsts c;
 };
 
-// one column by four slots of NT threads: the four forward transforms, the
+// one column (of the kl in use) by four slots of NT threads: the four forward transforms, the
 // spectral transposes, two inverse transforms
 template <int L, int NT>
 __device__ __forceinline__ void adj_col_body(const AdjColArgs &a, const double2 *__restrict__ twy, int bid, int nblk) {
@@ -495,13 +500,20 @@ __device__ __forceinline__ void adj_col_body(const AdjColArgs &a, const double2 
   double cx1 = 0.0, cy1 = 0.0, cx0 = 0.0, cy0 = 0.0, b10 = 0.0, b11 = 0.0;
   if (ab2) { cx1 = a.s->cx1; cy1 = a.s->cy1; cx0 = a.s->cx0; cy0 = a.s->cy0; b10 = a.s->b10; b11 = a.s->b11; }
   double2 lw[EL], ln[EL];
+  double dl[EL];
+  const double kx2 = (double)(kx * kx);
 #pragma unroll
   for (int q = 0; q < EL; ++q) {
     const int idx = tid + q * NTHR;
     lw[q] = ln[q] = make_double2(0.0, 0.0);
+    dl[q] = dealias_fast(c, kx, abs(ky_signed(idx, L)));  // 0: both are zero
     if (L % NTHR == 0 || idx < L) {
-      lw[q] = a.lW[(size_t)idx * H + kx];
-      if (ab2) ln[q] = a.lNL[(size_t)idx * H + kx];
+      const size_t g = (size_t)(dl[q] != 0.0 ? idx : 0) * H + kx;
+      const double2 w = a.lW[g], n = a.lNL[g];
+      if (dl[q] != 0.0) {
+        lw[q] = w;
+        if (ab2) ln[q] = n;
+      }
     }
   }
   {
@@ -524,7 +536,6 @@ __device__ __forceinline__ void adj_col_body(const AdjColArgs &a, const double2 
     grp_sync<WAVE>();
   }
   const bool same = cx0 == cx1 && cy0 == cy1;
-  const double rx = 1.0 / c.kxt2, ry = 1.0 / c.kyt2, kx2 = (double)(kx * kx);
 #pragma unroll
   for (int q = 0; q < EL; ++q) {
     const int idx = tid + q * NTHR;
@@ -554,7 +565,7 @@ __device__ __forceinline__ void adj_col_body(const AdjColArgs &a, const double2 
         l.y += div_by(lpsi.y, quot, rq);
       }
       const double v1 = exp(cx1 * kx2 + cy1 * ky2);
-      const double f = v1 * dealias_fast(c, kx, aky, rx, ry);
+      const double f = v1 * dl[q];
       lw0 = make_double2(f * l.x, f * l.y);
       lnl = make_double2(b10 * lw0.x + ln[q].x, b10 * lw0.y + ln[q].y);
       if (!a.explicit_step) {

@@ -155,12 +155,22 @@ __device__ __forceinline__ double div_by(double a, double b, double r) {
 
 // dealias(c, kx, ky) with the divisions left to the modes on the ellipse's
 // edge, where a product with the reciprocals could decide otherwise
-__device__ __forceinline__ double dealias_fast(const StepConsts &c, int kx, int ky, double rx, double ry) {
+__device__ __forceinline__ double dealias_fast(const StepConsts &c, int kx, int ky) {
   if (!c.idealis) return 1.0;
   const double a = (double)kx, b = (double)ky;
-  const double q = a * a * rx + b * b * ry;
+  const double q = a * a * c.rkxt2 + b * b * c.rkyt2;
   if (fabs(q - 1.0) < 1e-12) return dealias(c, kx, ky);
   return q >= 1.0 ? 0.0 : 1.0;
+}
+
+// Tile of workgroup bid when the first nl of nblk tiles are the ones with work
+// (the others' columns are beyond the dealiasing ellipse): as xcd_remap, but
+// each XCD gets its share of either kind.
+__device__ __forceinline__ int live_remap(int bid, int nblk, int nl) {
+  if (nblk % 8 != 0) return bid;
+  nl = min((nl + 7) & ~7, nblk);
+  const int x = bid & 7, i = bid >> 3, l = nl >> 3, d = (nblk - nl) >> 3;
+  return i < l ? x * l + i : nl + x * d + (i - l);
 }
 
 // One workgroup per TX columns, NS slots of TX*NT threads.  Slots 0 and 1
@@ -181,23 +191,29 @@ __device__ __forceinline__ void col_step_body(const ColStepArgs &a, const double
   const StepConsts &c = a.c;
   const int tid = threadIdx.x, H = c.H;
   const int slot = tid / (TX * NT), w = tid - slot * (TX * NT), cc = w % TX, t = w / TX;
-  const int kx0 = xcd_remap(bid, nblk) * TX;
+  const int kx0 = live_remap(bid, nblk, (c.kc + TX - 1) / TX) * TX;
   double2 *xb = lds + slot * SB + cc;
   const bool px_on = a.Rpx != nullptr;
   FftTw<L, NT> T;
   T.load(twy, 1, t);
   const double b10 = a.s->b10, b11 = a.s->b11, cx1 = a.s->cx1, cy1 = a.s->cy1, cx0 = a.s->cx0, cy0 = a.s->cy0;
-  // the update's own operands, in flight during the forward transforms
+  // the update's own operands, in flight during the forward transforms; a mode
+  // that dealiasing removes needs none
   const int c2 = tid % TX, kx = kx0 + c2, i0 = tid / TX;  // rows i0 + q NTHR/TX of column kx
   constexpr bool PREF = EL <= 2;
   double2 w0[EL], n1[EL];
+  double dl[EL];
   auto operands = [&](int q) {
     const int idx = i0 + q * (NTHR / TX);
     w0[q] = n1[q] = make_double2(0.0, 0.0);
+    dl[q] = kx < c.kc ? dealias_fast(c, kx, abs(ky_signed(idx, L))) : 0.0;
     if (L * TX % NTHR == 0 || idx < L) {
-      const size_t g = (size_t)idx * H + kx;
-      w0[q] = a.W0[g];
-      if (!a.explicit_step) n1[q] = a.NL1[g];
+      const size_t g = (size_t)(dl[q] != 0.0 ? idx : 0) * H + kx;
+      const double2 w = a.W0[g], n = a.explicit_step ? w : a.NL1[g];
+      if (dl[q] != 0.0) {
+        w0[q] = w;
+        if (!a.explicit_step) n1[q] = n;
+      }
     }
   };
   if constexpr (PREF) {
@@ -231,7 +247,6 @@ __device__ __forceinline__ void col_step_body(const ColStepArgs &a, const double
   {
     // a constant time step: both viscous factors are the same number
     const bool same = cx0 == cx1 && cy0 == cy1;
-    const double rx = 1.0 / c.kxt2, ry = 1.0 / c.kyt2;
     const double kx2 = (double)(kx * kx);
     if constexpr (!PREF) {
 #pragma unroll
@@ -254,7 +269,7 @@ __device__ __forceinline__ void col_step_body(const ColStepArgs &a, const double
           nl = make_double2(Fc.x + kyf * Fp.y, Fc.y - kyf * Fp.x);
           const double ky2 = (double)(aky * aky);
           const double v1 = exp(cx1 * kx2 + cy1 * ky2);
-          const double d = dealias_fast(c, kx, aky, rx, ry);
+          const double d = dl[q];
           if (a.explicit_step) {
             w1.x = (w0[q].x + b10 * nl.x) * v1 * d;
             w1.y = (w0[q].y + b10 * nl.y) * v1 * d;
@@ -277,6 +292,7 @@ __device__ __forceinline__ void col_step_body(const ColStepArgs &a, const double
       }
     }
   }
+  if (kx0 >= c.kc) return;  // vorticity and everything derived from it are zero, and not read
   // the derived fields, NS at a time: written to the slots' buffers by the
   // threads that hold the update, transformed back and stored
   auto derived = [&](int f, int q) {
@@ -337,7 +353,7 @@ __device__ __forceinline__ void col_direct_body(const ColStepArgs &a, const doub
   static_assert(Out::M == NT && M0 % NT == 0, "values stay in their thread");
   const StepConsts &c = a.c;
   const int tid = threadIdx.x, H = c.H, cc = tid % TX, t = tid / TX;
-  const int kx = xcd_remap(bid, nblk) * TX + cc;
+  const int kx = live_remap(bid, nblk, (c.kc + TX - 1) / TX) * TX + cc;
   double2 *xb = lds + cc;
   FftTw<L, NT> T;
   T.load(twy, 1, t);
@@ -355,7 +371,7 @@ __device__ __forceinline__ void col_direct_body(const ColStepArgs &a, const doub
   {
     const double b10 = a.s->b10, b11 = a.s->b11, cx1 = a.s->cx1, cy1 = a.s->cy1, cx0 = a.s->cx0, cy0 = a.s->cy0;
     const bool same = cx0 == cx1 && cy0 == cy1;
-    const double rx = 1.0 / c.kxt2, ry = 1.0 / c.kyt2, kx2 = (double)(kx * kx);
+    const double kx2 = (double)(kx * kx);
 #pragma unroll
     for (int q = 0; q < E; ++q) {
       if (q % 2 == 0) __builtin_amdgcn_sched_barrier(0);
@@ -372,14 +388,15 @@ __device__ __forceinline__ void col_direct_body(const ColStepArgs &a, const doub
         nl = make_double2(Fc.x + kyf * Fp.y, Fc.y - kyf * Fp.x);
         const double ky2 = (double)(aky * aky);
         const double v1 = exp(cx1 * kx2 + cy1 * ky2);
-        const double d = dealias_fast(c, kx, aky, rx, ry);
-        const double2 w0 = a.W0[g];
+        const double d = kx < c.kc ? dealias_fast(c, kx, aky) : 0.0;
+        const double2 zero = make_double2(0.0, 0.0);  // a mode that dealiasing removes needs no operands
+        const double2 w0 = d != 0.0 ? a.W0[g] : zero;
         if (a.explicit_step) {
           w1.x = (w0.x + b10 * nl.x) * v1 * d;
           w1.y = (w0.y + b10 * nl.y) * v1 * d;
         } else {
           const double v0 = same ? v1 : exp(cx0 * kx2 + cy0 * ky2);
-          const double2 n1 = a.NL1[g];
+          const double2 n1 = d != 0.0 ? a.NL1[g] : zero;
           const double2 n1v = make_double2(n1.x * v0, n1.y * v0);
           w1.x = ((w0.x + b10 * nl.x) + b11 * n1v.x) * v1 * d;
           w1.y = ((w0.y + b10 * nl.y) + b11 * n1v.y) * v1 * d;
@@ -390,6 +407,7 @@ __device__ __forceinline__ void col_direct_body(const ColStepArgs &a, const doub
       W[q] = w1;
     }
   }
+  if (kx - cc >= c.kc) return;  // vorticity and everything derived from it are zero, and not read
   // omega, i ky omega, then W becomes psi: psi, i ky psi, -ky^2 psi
 #pragma unroll
   for (int k = 0; k < 5; ++k) {
@@ -640,11 +658,12 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
     const double2 *src = slot == 0 ? a.Cpsiy : slot == 1 ? a.Cpsi : (FIVE && slot == 4) ? a.Cwy : a.Cw;
     const bool ik = slot == 1 || slot == 3;
     src += rowk;
+    const int kc = a.c.kc;
     fft_io<H, NT, true, 1, WAVE, LEAN, LEAN ? 4 : 16>(
         xb, T, t, NEXT || slot < 3,
         [&](int, int, int e) {
           const int q = e == 0 ? 0 : H - e;
-          double2 xa = src[e], xq = src[q];
+          double2 xa = live(src, e, H, kc), xq = live(src, q, H, kc);
           if (ik) { xa = mul_ik(xa, (double)e * sx); xq = mul_ik(xq, (double)q * sx); }
           return c2r_elem(xa, xq, e, cconj(twx[e]));
         },
@@ -821,7 +840,8 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
     if (inv) {
       for_in([&](int q, int e) {
         if (LEAN && q % 2 == 0) __builtin_amdgcn_sched_barrier(0);
-        in[q] = cconj(c2r_elem(a.Cwy[rowk + e], a.Cwy[rowk + (e == 0 ? 0 : H - e)], e, cconj(twx[e])));
+        in[q] = cconj(c2r_elem(live(a.Cwy + rowk, e, H, a.c.kc),
+                               live(a.Cwy + rowk, e == 0 ? 0 : H - e, H, a.c.kc), e, cconj(twx[e])));
       });
     } else if (act) {
       for_in([&](int q, int e) { in[q] = xb[pidx(e)]; });
