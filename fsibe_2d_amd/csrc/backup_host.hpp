@@ -407,12 +407,7 @@ extern "C" int fsibe_inicond_read(fsibe_sim *s, const char *path) {
   HIPCHK(hipStreamSynchronize(s->stream));
   HIPCHK(hipMemcpyAsync(s->fb_sa, v.data(), sizeof(double) * N, hipMemcpyHostToDevice, s->stream));
   CHK(rows_r2c(s->nx, s->ny, s->px, s->twx, s->fb_sa, s->T[6], s->stream));
-  const double norm = 1.0 / ((double)s->nx * (double)s->ny);
-  CHK(with_cols<1>(s->py, s->H, pick_tx(s->H, s->ny, 1, 1), [&](auto F, int nt, int TX) -> int {
-    const size_t lds = sizeof(double2) * TX * padlen(s->ny);
-    KLAUNCH(k_cols_fwd_pack<decltype(F)>, s->H / TX, nt, lds, s->stream, s->T[6], s->fb_p, F, s->twy, s->H, norm);
-    return FSIBE_OK;
-  }));
+  CHK(cols_pack(s->H, s->ny, s->py, s->twy, s->T[6], s->fb_p, s->stream));
   k_packed_to_half<<<grid1d((size_t)s->H * (s->ny / 2)), 256, 0, s->stream>>>(s->fb_p, s->W[0], s->nx, s->ny);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s->stream));

@@ -32,6 +32,7 @@
 #include "kernels_mask.hpp"
 #include "kernels_step.hpp"
 #include "kernels_fused.hpp"
+#include "kernels_spectral.hpp"
 #include "transfer.hpp"
 #include "kernels_adjoint.hpp"
 #include "kinematics.hpp"
@@ -508,42 +509,163 @@ extern "C" int fsibe_spectral_destroy(fsibe_spectral *c) {
 }
 
 // real rows -> half spectrum (unnormalised)
+// fn(shape) for row transforms of H complex values; false if there is none.
+// Threads and rows per workgroup as measured (kernels_spectral.hpp): about H/8
+// threads a row, more where that leaves the last pass uneven.
+template <class Fn>
+static bool with_rows_io(int H, Fn &&fn) {
+  switch (H) {
+    case 32: fn(RowsShape<32, 8, 8>{}); return true;
+    case 48: fn(RowsShape<48, 16, 4>{}); return true;
+    case 64: fn(RowsShape<64, 16, 4>{}); return true;
+    case 96: fn(RowsShape<96, 32, 2>{}); return true;
+    case 128: fn(RowsShape<128, 32, 2>{}); return true;
+    case 192: fn(RowsShape<192, 32, 2>{}); return true;
+    case 256: fn(RowsShape<256, 64, 1>{}); return true;
+    case 384: fn(RowsShape<384, 64, 1>{}); return true;
+    case 512: fn(RowsShape<512, 64, 1>{}); return true;
+    case 768: fn(RowsShape<768, 256, 1>{}); return true;
+    case 1024: fn(RowsShape<1024, 128, 1>{}); return true;
+    default: return false;
+  }
+}
+// fixed-length row policies whose length always has such a shape
+constexpr bool always_rows_io(int H) {
+  return H == 64 || H == 128 || H == 192 || H == 256 || H == 384 || H == 512 || H == 1024;
+}
+
+// fn(shape) for column transforms of ny values; false if there is none.  Two
+// columns per workgroup, except where four were faster (384: 17.2 against
+// 20.0 us for both directions of 384^2).
+template <class Fn>
+static bool with_cols_io(int ny, int H, Fn &&fn) {
+  if (H % 4 == 0 && ny == 384) { fn(ColsShape<384, 4, 48>{}); return true; }
+  if (H % 2) return false;
+  switch (ny) {
+    case 64: fn(ColsShape<64, 2, 16>{}); return true;
+    case 96: fn(ColsShape<96, 2, 24>{}); return true;
+    case 128: fn(ColsShape<128, 2, 32>{}); return true;
+    case 192: fn(ColsShape<192, 2, 24>{}); return true;
+    case 256: fn(ColsShape<256, 2, 32>{}); return true;
+    case 512: fn(ColsShape<512, 2, 64>{}); return true;
+    case 768: fn(ColsShape<768, 2, 96>{}); return true;
+    case 1024: fn(ColsShape<1024, 2, 128>{}); return true;
+    case 1536: fn(ColsShape<1536, 2, 192>{}); return true;
+    case 2048: fn(ColsShape<2048, 2, 256>{}); return true;
+    default: return false;
+  }
+}
+
+// fn(shape) for a grid of up to 2048 half-spectrum entries in one workgroup;
+// false if there is none
+template <class Fn>
+static bool with_small(int H, int ny, Fn &&fn) {
+  if (H == 32 && ny == 64) { fn(SmallShape<32, 64, 4, 8, 512>{}); return true; }
+  if (H == 64 && ny == 32) { fn(SmallShape<64, 32, 8, 4, 512>{}); return true; }
+  if (H == 32 && ny == 32) { fn(SmallShape<32, 32, 4, 4, 256>{}); return true; }
+  return false;
+}
+
 static int rows_r2c(int nx, int ny, const FftPlan &px, const double2 *twx, const double *f, double2 *out,
                     hipStream_t st) {
+  int rc = FSIBE_OK;
+  if (with_rows_io(nx / 2, [&](auto S) {
+        using ST = decltype(S);
+        rc = [&]() -> int {
+          KLAUNCH(k_rows_fwd<ST>, (ny + ST::RPB - 1) / ST::RPB, ST::THREADS, ST::LDS, st, f, out, twx, ny);
+          return FSIBE_OK;
+        }();
+      }))
+    return rc;
   const size_t lds = sizeof(double2) * padlen(nx / 2);
   return with_rows<1>(px, [&](auto F, int nt) -> int {
-    KLAUNCH(k_rows_r2c<decltype(F)>, ny, nt, lds, st, f, out, F, twx);
+    if constexpr (!always_rows_io(fixed_len<decltype(F)>::v)) KLAUNCH(k_rows_r2c<decltype(F)>, ny, nt, lds, st, f, out, F, twx);
     return FSIBE_OK;
   });
 }
 
 static int rows_c2r(int nx, int ny, const FftPlan &px, const double2 *twx, const double2 *in, double *f,
                     hipStream_t st) {
+  int rc = FSIBE_OK;
+  if (with_rows_io(nx / 2, [&](auto S) {
+        using ST = decltype(S);
+        rc = [&]() -> int {
+          KLAUNCH(k_rows_inv<ST>, (ny + ST::RPB - 1) / ST::RPB, ST::THREADS, ST::LDS, st, in, f, twx, ny);
+          return FSIBE_OK;
+        }();
+      }))
+    return rc;
   const size_t lds = sizeof(double2) * padlen(nx / 2);
   return with_rows<1>(px, [&](auto F, int nt) -> int {
-    KLAUNCH(k_rows_c2r<decltype(F)>, ny, nt, lds, st, in, f, F, twx);
+    if constexpr (!always_rows_io(fixed_len<decltype(F)>::v)) KLAUNCH(k_rows_c2r<decltype(F)>, ny, nt, lds, st, in, f, F, twx);
+    return FSIBE_OK;
+  });
+}
+
+// columns of the half spectrum in -> packed layout, and back
+static int cols_pack(int H, int ny, const FftPlan &py, const double2 *twy, const double2 *in, double *fk,
+                     hipStream_t st) {
+  const double norm = 1.0 / ((double)(2 * H) * (double)ny);
+  int rc = FSIBE_OK;
+  if (with_cols_io(ny, H, [&](auto S) {
+        using ST = decltype(S);
+        rc = [&]() -> int {
+          KLAUNCH(k_cols_fwd<ST>, H / ST::TX, ST::THREADS, ST::LDS, st, in, fk, twy, H, norm);
+          return FSIBE_OK;
+        }();
+      }))
+    return rc;
+  return with_cols<1>(py, H, pick_tx(H, ny, 1, 1), [&](auto F, int nt, int TX) -> int {
+    const size_t lds = sizeof(double2) * TX * padlen(ny);
+    KLAUNCH(k_cols_fwd_pack<decltype(F)>, H / TX, nt, lds, st, in, fk, F, twy, H, norm);
+    return FSIBE_OK;
+  });
+}
+static int cols_unpack(int H, int ny, const FftPlan &py, const double2 *twy, const double *fk, double2 *out,
+                       hipStream_t st) {
+  int rc = FSIBE_OK;
+  if (with_cols_io(ny, H, [&](auto S) {
+        using ST = decltype(S);
+        rc = [&]() -> int {
+          KLAUNCH(k_cols_inv<ST>, H / ST::TX, ST::THREADS, ST::LDS, st, fk, out, twy, H);
+          return FSIBE_OK;
+        }();
+      }))
+    return rc;
+  return with_cols<1>(py, H, pick_tx(H, ny, 1, 1), [&](auto F, int nt, int TX) -> int {
+    const size_t lds = sizeof(double2) * TX * padlen(ny);
+    KLAUNCH(k_cols_unpack_inv<decltype(F)>, H / TX, nt, lds, st, fk, out, F, twy, H);
     return FSIBE_OK;
   });
 }
 
 static int dev_coftxy(fsibe_spectral *c, const double *f, double *fk, hipStream_t st) {
+  int rc = FSIBE_OK;
+  if (with_small(c->H, c->ny, [&](auto S) {
+        using ST = decltype(S);
+        rc = [&]() -> int {
+          KLAUNCH(k_fwd2d<ST>, 1, ST::THREADS, ST::LDSF, st, f, fk, c->twx, c->twy,
+                  1.0 / ((double)c->nx * (double)c->ny));
+          return FSIBE_OK;
+        }();
+      }))
+    return rc;
   CHK(rows_r2c(c->nx, c->ny, c->px, c->twx, f, c->tmp, st));
-  const double norm = 1.0 / ((double)c->nx * (double)c->ny);
-  return with_cols<1>(c->py, c->H, pick_tx(c->H, c->ny, 1, 1), [&](auto F, int nt, int TX) -> int {
-    const size_t lds = sizeof(double2) * TX * padlen(c->ny);
-    KLAUNCH(k_cols_fwd_pack<decltype(F)>, c->H / TX, nt, lds, st, c->tmp, fk, F, c->twy, c->H, norm);
-    return FSIBE_OK;
-  });
+  return cols_pack(c->H, c->ny, c->py, c->twy, c->tmp, fk, st);
 }
 
 static int dev_cofitxy(fsibe_spectral *c, const double *fk, double *f, hipStream_t st) {
-  CHK(with_cols<1>(c->py, c->H, pick_tx(c->H, c->ny, 1, 1), [&](auto F, int nt, int TX) -> int {
-    const size_t lds = sizeof(double2) * TX * padlen(c->ny);
-    KLAUNCH(k_cols_unpack_inv<decltype(F)>, c->H / TX, nt, lds, st, fk, c->tmp, F, c->twy, c->H);
-    return FSIBE_OK;
-  }));
-  CHK(rows_c2r(c->nx, c->ny, c->px, c->twx, c->tmp, f, st));
-  return FSIBE_OK;
+  int rc = FSIBE_OK;
+  if (with_small(c->H, c->ny, [&](auto S) {
+        using ST = decltype(S);
+        rc = [&]() -> int {
+          KLAUNCH(k_inv2d<ST>, 1, ST::THREADS, ST::LDSI, st, fk, f, c->twx, c->twy);
+          return FSIBE_OK;
+        }();
+      }))
+    return rc;
+  CHK(cols_unpack(c->H, c->ny, c->py, c->twy, fk, c->tmp, st));
+  return rows_c2r(c->nx, c->ny, c->px, c->twx, c->tmp, f, st);
 }
 
 static int grid1d(size_t n) { return (int)std::min<size_t>((n + 255) / 256, 4096); }
@@ -665,13 +787,7 @@ extern "C" int fsibe_dev_coftxy_noalloc(int nx, int ny, const double *d_f, doubl
     }
   }
   CHK(rows_r2c(nx, ny, px, twx, d_f, tmp, st));
-  const int H = nx / 2;
-  const double norm = 1.0 / ((double)nx * (double)ny);
-  return with_cols<1>(py, H, pick_tx(H, ny, 1, 1), [&](auto F, int nt, int TX) -> int {
-    const size_t lds = sizeof(double2) * TX * padlen(ny);
-    KLAUNCH(k_cols_fwd_pack<decltype(F)>, H / TX, nt, lds, st, tmp, d_fk, F, twy, H, norm);
-    return FSIBE_OK;
-  });
+  return cols_pack(nx / 2, ny, py, twy, tmp, d_fk, st);
 }
 
 // host-pointer wrappers: copy in, run, copy out
