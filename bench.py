@@ -24,6 +24,7 @@ from __future__ import annotations
 import argparse
 import ctypes as C
 import json
+import math
 import os
 import re
 import sys
@@ -52,9 +53,14 @@ def alg_bytes(name: str, nx: int, ny: int, visc: bool, box_rows: int, box_cols: 
         "create_mask": 3 * 8.0 * mask_px,           # mask, mask_vx, mask_vy on the mask box
         "cols_vortk_n0": 3 * S,                     # W0 -> A, B
         "rows_nonlinear": 7 * S,                    # A, B, u1, u2, chi_s -> Rc, Rpx
-        "cols_ab2_update": 6 * S,                   # Rc, Rpx, W0, nlk(n1) -> nlk(n0), W1
-        "cols_vortk_n1": (5 if visc else 4) * S,    # W1 -> omega, psi, i ky psi (, -ky^2 psi)
-        "rows_velocity_pressure": 9 * S,            # 3 inputs + vor_mean r/w -> u1, u2, Rq, Rqy
+        # the fused column stage: Rc, Rpx (box rows), W0 and nlk(n1) inside the
+        # dealiasing ellipse (pi/9 of the modes) -> nlk(n0), W1, and on the
+        # two thirds of the columns that reach it omega, psi, i ky psi
+        # (, -ky^2 psi on the box rows)
+        "cols_ab2_update": (1 + 2 * math.pi / 9 + 2 + 2) * S + box_rows * rowS * (1 + (2 / 3 if visc else 0)),
+        "cols_vortk_n1": (5 if visc else 4) * S,    # launched only where no fused column stage exists
+        # 3 inputs (two thirds of their columns) + vor_mean r/w -> u1, u2, Rq, Rqy
+        "rows_velocity_pressure": 8 * S,
         "cols_pressure": 2 * S + box_rows * rowS,   # Rq, Rqy -> q on the beam rows
         "rows_pressure_box": box_rows * rowS * (6 if visc else 3) + 3 * 8.0 * box_rows * box_cols,
     }.get(name, 0.0)
@@ -72,8 +78,8 @@ def hip_sync():
 
 # kernel names in rocprofv3 output for each class of fsibe_profile_read
 ROCPROF_NAME = {"cols_vortk_n0": "k_cols_inv_fields", "rows_nonlinear": "k_rows_nl",
-                "cols_ab2_update": "k_cols_ab2", "cols_vortk_n1": "k_cols_inv_fields",
-                "rows_velocity_pressure": "k_rows_press", "cols_pressure": "k_cols_press",
+                "cols_ab2_update": "k_col_step", "cols_vortk_n1": "k_cols_inv_fields",
+                "rows_velocity_pressure": "k_row_step", "cols_pressure": "k_press_step",
                 "rows_pressure_box": "k_rows_box", "create_mask": "k_mask", "delta_interp_forces": "k_forces"}
 
 

@@ -1220,7 +1220,7 @@ struct fsibe_sim {
   Window win[2];  // cal_drag's window per beam
   int nprim = 0, ntg = 0;
   size_t off_prim = 0, off_beam = 0, off_tg = 0, off_nd = 0, off_cd = 0, off_val = 0;
-  int nprim_cap = 0;  // room for mask primitives in the staging buffer (and the mask kernel's LDS)
+  int nprim_cap = 0;  // room for mask primitives in the staging buffer
   ForceGeom fg;
   bool forces_ready = false;
   bool press_box_valid = false;
