@@ -305,7 +305,7 @@ __device__ __forceinline__ void col_step_body(const ColStepArgs &a, const double
   };
 #pragma unroll
   for (int rd = 0; rd < (4 + NS) / NS; ++rd) {
-    // the fields of this round: omega, psi, i ky psi, -ky^2 psi, i ky omega
+    // the fields of this turn: omega, psi, i ky psi, -ky^2 psi, i ky omega
     // in this order for four slots; for two (omega, psi), (i ky psi, i ky
     // omega), (-ky^2 psi)
     constexpr int kF[5] = {0, 1, 2, NS == 2 ? 4 : 3, NS == 2 ? 3 : 4};
