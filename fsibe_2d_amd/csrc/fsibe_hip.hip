@@ -3445,8 +3445,9 @@ static int tune_launch(const fsibe_batch *b, const BatchGroup &g, int k, ColSel 
 // launches each after a warm-up launch, and the fastest is kept; the single
 // path's choice stays unless another is more than 2 % faster.  No choice
 // changes a result (ColSel), so the members stay bit-identical to their own
-// runs whatever the measurements say.
-static int tune_batch(fsibe_batch *b) {
+// runs whatever the measurements say.  Stages whose bit is set in `skip` keep
+// their static choice untimed.
+static int tune_batch(fsibe_batch *b, unsigned skip = 0) {
   for (fsibe_sim *s : b->m) HIPCHK(hipStreamSynchronize(s->stream));
   size_t bytes = 0;
   for (auto &g : b->groups)
@@ -3466,6 +3467,7 @@ static int tune_batch(fsibe_batch *b) {
       break;
     }
     for (int k : kColStages) {
+      if (skip >> k & 1u) continue;
       const int bm = (k == B_K4 || k == B_K7) ? 2 : 1;
       std::vector<ColSel> cand;
       for (int ct = 1; ct >= 0; --ct)
@@ -3545,7 +3547,12 @@ static int sim_tune_cols(fsibe_sim *s) {
     g.sel[B_K5] = static_sel(s, 1, nf5);
     g.sel[B_K7] = static_sel(s, 2, 1);
     t.groups.push_back(g);
-    const int rc = tune_batch(&t);
+    // only what this grid launches: K4, K5 and K7 are not where the fused
+    // column stage and the pressure stage replace them
+    unsigned skip = 0;
+    if (with_col_step(s->ny, s->H, s->penal_on, [](auto) {})) skip |= 1u << B_K4 | 1u << B_K5;
+    if (with_press_step(s->ny, s->H, [](auto) {})) skip |= 1u << B_K7;
+    const int rc = tune_batch(&t, skip);
     const std::array<ColSel, 4> sel{t.groups[0].sel[B_K1], t.groups[0].sel[B_K4], t.groups[0].sel[B_K5],
                                     t.groups[0].sel[B_K7]};
     t.groups[0].stream = nullptr;
