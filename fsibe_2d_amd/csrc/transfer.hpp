@@ -14,6 +14,13 @@
 // already knows (pinned, managed or device memory), takes the runtime's path,
 // as does one of less than 4 MiB (1.2 MB: 90 us by the runtime, 180 us here,
 // where waking the threads and a call per chunk cost more than they save).
+//
+// The threads are joined when the process ends normally or the library is
+// unloaded; later copies (by destructors that run after that) take the
+// runtime's path, as do those of a forked child, which has the ring but none
+// of the threads.  The object itself is never destroyed: a condition variable
+// that threads of the parent wait on must not be destroyed in the child (the
+// destructor waits for them), and late callers may still use the rest.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <unistd.h>
@@ -32,29 +39,37 @@ namespace fsibe {
 class Transfer {
  public:
   static Transfer &get() {
-    static Transfer t;
-    return t;
+    static Transfer *t = new Transfer;
+    static struct End {
+      ~End() { t->stop(); }
+    } end;
+    return *t;
   }
   // download returns when the data are in place; upload when the source may be
   // reused, or, where the runtime's path is taken, as hipMemcpyAsync does
   hipError_t download(void *dst, const void *src, size_t bytes, hipStream_t st) { return copy(dst, src, bytes, st, false); }
   hipError_t upload(void *dst, const void *src, size_t bytes, hipStream_t st) { return copy(dst, src, bytes, st, true); }
 
-  ~Transfer() {
-    if (pid_ != getpid()) {  // a forked child: the threads are not there
-      new std::vector<std::thread>(std::move(workers_));
-      return;
-    }
+ private:
+  Transfer() = default;
+
+  // ends the helpers; the pinned ring stays until the process ends (the
+  // runtime may be gone)
+  void stop() {
+    if (pid_ != getpid()) return;  // a forked child: the threads are not there
+    // held by a copy of another thread that the process's end cuts short: its
+    // helpers end with the process
+    std::unique_lock<std::mutex> use(use_, std::try_to_lock);
+    if (!use.owns_lock()) return;
     {
       std::lock_guard<std::mutex> g(mu_);
       stop_ = true;
     }
     cv_.notify_all();
     for (auto &w : workers_) w.join();
-    // the pinned ring stays until the process ends: the runtime may be gone
+    workers_.clear();
   }
 
- private:
   static constexpr size_t kMin = 4 << 20;
   static constexpr size_t kSlot = 2 << 20;  // largest chunk: a huge page, faulted in by one thread
   static constexpr int kSlots = 16, kHelpers = 7;
@@ -65,8 +80,9 @@ class Transfer {
   }
 
   // the ring and the helpers, made at the first use (also while some other
-  // thread captures a graph)
+  // thread captures a graph); the caller holds use_
   bool ready() {
+    if (stop_) return false;
     if (ring_) return pid_ == getpid();
     if (failed_) return false;
     failed_ = true;
