@@ -11,9 +11,14 @@
 // One ring and one pool of threads per process, made at the first large
 // copy: 32 MiB pinned and at most 7 threads, asleep between copies.  A copy
 // that finds them in use by another thread, or whose host pointer the runtime
-// already knows (pinned, managed or device memory), takes the runtime's path,
-// as does one of less than 4 MiB (1.2 MB: 90 us by the runtime, 180 us here,
-// where waking the threads and a call per chunk cost more than they save).
+// already knows (pinned, managed or device memory), takes the runtime's path.
+// So does a download of less than 8 MiB or an upload of less than 48 MiB, where
+// waking the threads and a call per chunk cost more than they save: the
+// runtime copies from the device into memory at 8 to 19 GB/s but reads resident
+// memory at 30.  Both paths measured, us by the runtime and here: downloads
+// of 4.5 MiB 270 / 288, 6 MiB 364 / 364, 8 MiB 482 / 407, 32 MiB 1950 / 963 (into
+// fresh memory 3460 / 1230), 128 MiB 7770 / 3470; uploads of 4.5 MiB 176 / 294,
+// 8 MiB 268 / 427, 32 MiB 1006 / 1034, 48 MiB 1735 / 1493, 64 MiB 2420 / 1911, 128 MiB 4706 / 3599.
 //
 // The threads are joined when the process ends normally or the library is
 // unloaded; later copies (by destructors that run after that) take the
@@ -70,7 +75,7 @@ class Transfer {
     workers_.clear();
   }
 
-  static constexpr size_t kMin = 4 << 20;
+  static constexpr size_t kMinDown = (size_t)8 << 20, kMinUp = (size_t)48 << 20;
   static constexpr size_t kSlot = 2 << 20;  // largest chunk: a huge page, faulted in by one thread
   static constexpr int kSlots = 16, kHelpers = 7;
 
@@ -108,7 +113,7 @@ class Transfer {
   }
 
   hipError_t copy(void *dst, const void *src, size_t bytes, hipStream_t st, bool up) {
-    if (bytes < kMin) return plain(dst, src, bytes, st, up);
+    if (bytes < (up ? kMinUp : kMinDown)) return plain(dst, src, bytes, st, up);
     hipPointerAttribute_t at;
     const hipError_t known = hipPointerGetAttributes(&at, up ? src : dst);
     if (known != hipSuccess) (void)hipGetLastError();

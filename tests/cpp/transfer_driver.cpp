@@ -14,8 +14,10 @@
 
 // ---- stand-ins -------------------------------------------------------------
 static void (*on_query)() = nullptr;  // called once, by the next event query
+static int copies = 0;                // hipMemcpyAsync calls
 extern "C" {
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t) {
+  ++copies;
   memcpy(dst, src, n);
   return hipSuccess;
 }
@@ -82,10 +84,25 @@ int main(int argc, char **argv) {
   const std::string c = argc > 1 ? argv[1] : "";
   constexpr size_t kBig = (size_t)9 << 20;
   if (c == "sizes") {
-    for (size_t n : {(size_t)1, (size_t)4194303, (size_t)4194304, (size_t)4194305, kBig + 3, (size_t)70 << 20})
+    const size_t d = (size_t)8 << 20, u = (size_t)48 << 20;
+    for (size_t n : {(size_t)1, d - 1, d, d + 1, kBig + 3, u - 1, u, u + 1, (size_t)70 << 20})
       if (!round_trip(n)) return std::printf("%zu bytes differ\n", n), 1;
     std::puts("equal");
     return 0;
+  }
+  if (c == "lines") {  // the runtime's path (one copy) below each direction's line, chunks from there on
+    std::vector<char> a((size_t)48 << 20), b(a.size());
+    auto count = [&](bool up, size_t n) {
+      copies = 0;
+      auto &t = fsibe::Transfer::get();
+      (void)(up ? t.upload(a.data(), b.data(), n, nullptr) : t.download(a.data(), b.data(), n, nullptr));
+      return copies;
+    };
+    const size_t d = (size_t)8 << 20, u = a.size();
+    const bool ok = count(false, (size_t)6 << 20) == 1 && count(false, d - 1) == 1 && count(false, d) > 1 &&
+                    count(true, d) == 1 && count(true, (size_t)32 << 20) == 1 && count(true, u - 1) == 1 && count(true, u) > 1;
+    std::puts(ok ? "as measured" : "another line");
+    return ok ? 0 : 1;
   }
   if (c == "late") {
     late.on = true;

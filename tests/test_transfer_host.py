@@ -1,5 +1,6 @@
-"""The threads behind the large host copies (fsibe_2d_amd/csrc/transfer.hpp)
-when the process forks or ends: a forked child, which has none of them, ends
+"""The large host copies (fsibe_2d_amd/csrc/transfer.hpp): what arrives, from
+which size in each direction they replace the runtime's, and their threads when
+the process forks or ends: a forked child, which has none of them, ends
 normally, and a copy that a late destructor makes still arrives.  Compiled with
 g++ on stand-ins for the HIP calls, so it runs with no GPU."""
 import os
@@ -20,7 +21,7 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["sizes", "fork", "fork_inside", "late"])
+@pytest.mark.parametrize("case", ["sizes", "lines", "fork", "fork_inside", "late"])
 def test_copies_threads_and_process_ends(driver, case):
     r = subprocess.run([driver, case], capture_output=True, text=True, timeout=60)
     print(case, r.returncode, r.stdout, r.stderr)
