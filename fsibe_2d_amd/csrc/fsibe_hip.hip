@@ -368,9 +368,17 @@ static bool size_ok(int nx, int ny) {
 // simulation, K4 + K5 with four fields + the dw/dy column of K1, us):
 // 256^2 19.0 -> 7.2, 384^2 22.9 -> 11.3, 512^2 21.3 -> 11.7, 768^2 30.7 ->
 // 22.1, 1024^2 37.9 -> 26.0, 2048^2 131 -> 125.
+// Columns of 4096 points, where px leaves no room: two columns a workgroup
+// with their fields one after another are too few workgroups below 192
+// columns, where the separate stages spread the fields over more.  A step of a
+// flow without a body, with the stages separate and fused, us: 64 columns 104
+// and 113 (one step a call: 127 and 144), 128 columns 127 and 129 (151 and
+// 160), 192 columns 139 and 127 (163 and 158).  next: the next step's terms are
+// formed too, which pays below 192 columns as well where the rows would need a
+// run-time plan for them (32 columns 108 and 85, 96: 138 and 102, 108: 177
+// and 157; 16 and 24: 200 and 204, 139 and 143).
 template <class Fn>
-static bool with_col_step(int ny, int H, bool px, Fn &&fn) {
-  (void)px;
+static bool with_col_step(int ny, int H, bool px, bool next, Fn &&fn) {
   switch (ny) {
     case 64: fn(ColStepShape<64, 1, 8, 4, false>{}); return true;
     case 96: fn(ColStepShape<96, 1, 12, 4, false>{}); return true;
@@ -391,7 +399,7 @@ static bool with_col_step(int ny, int H, bool px, Fn &&fn) {
       else fn(ColStepShape<2048, 2, 256, 0, false>{});
       return true;
     case 4096:
-      if (px) return false;
+      if (px || (H < 192 && !(next && H >= 32 && H != 64 && H != 128))) return false;
       fn(ColStepShape<4096, 2, 512, 0, false>{});
       return true;
     default: return false;
@@ -2485,7 +2493,7 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
   next = next && !sp10 && s->p.iMeanVelocity != 11;
   int rc = FSIBE_OK;
   PROF_BEGIN(s, P_COLS_AB2);
-  const bool fused_cols = with_col_step(s->ny, s->H, s->penal_on, [&](auto S) {
+  const bool fused_cols = with_col_step(s->ny, s->H, s->penal_on, next, [&](auto S) {
     using ST = decltype(S);
     rc = [&]() -> int {
       KLAUNCH(k_col_step<ST>, s->H / ST::TX, ST::THREADS, ST::LDS, s->stream,
@@ -3550,7 +3558,7 @@ static int sim_tune_cols(fsibe_sim *s) {
     // only what this grid launches: K4, K5 and K7 are not where the fused
     // column stage and the pressure stage replace them
     unsigned skip = 0;
-    if (with_col_step(s->ny, s->H, s->penal_on, [](auto) {})) skip |= 1u << B_K4 | 1u << B_K5;
+    if (with_col_step(s->ny, s->H, s->penal_on, false, [](auto) {})) skip |= 1u << B_K4 | 1u << B_K5;
     if (with_press_step(s->ny, s->H, [](auto) {})) skip |= 1u << B_K7;
     const int rc = tune_batch(&t, skip);
     const std::array<ColSel, 4> sel{t.groups[0].sel[B_K1], t.groups[0].sel[B_K4], t.groups[0].sel[B_K5],
