@@ -433,11 +433,15 @@ template <class F> struct fixed_len { static constexpr int v = 0; };
 template <int H, int NT> struct fixed_len<RowCT<H, NT>> { static constexpr int v = H; };
 template <int NY, int TX, int NT> struct fixed_len<ColCT<NY, TX, NT>> { static constexpr int v = NY; };
 constexpr bool always_col_step(int ny) { return ny == 128 || ny == 256 || ny == 384 || ny == 512; }
-constexpr bool always_row_step(int H) { return H == 128 || H == 192 || H == 256 || H == 512; }
+constexpr bool always_row_step(int H) { return H == 192 || H == 256 || H == 512; }
 
-// fn(shape) for the fused row stage (K6 and the convective part of the next
-// K2) of rows of H complex values on ny rows; false if there is none
-template <class Fn>
+// fn(shape) for the fused row stage (K6 and, with NEXT, the convective part of
+// the next K2) of rows of H complex values on ny rows; false if there is none.
+// Rows of 128 without NEXT: the stage's one wave a row, of which a quarter
+// has no transform then, against K6 alone, us, 256, 1024, 2048 and 4096 rows:
+// 8.3, 11.1, 16.5, 25.4 and 7.3, 9.5, 14.8, 23.6; with the pressure 11.6, 15.2, 20.8,
+// 31.0 and 11.4, 14.5, 20.6, 25.2.
+template <bool NEXT, class Fn>
 static bool with_row_step(int H, int ny, Fn &&fn) {
   switch (H) {
     case 32:
@@ -449,7 +453,9 @@ static bool with_row_step(int H, int ny, Fn &&fn) {
       fn(RowStepShape<64, 8, 4, 2, false>{});
       return true;
     case 96: fn(RowStepShape<96, 16, 4, 1, false>{}); return true;
-    case 128: fn(RowStepShape<128, 16, 4, 1, false>{}); return true;
+    case 128:
+      if constexpr (NEXT) fn(RowStepShape<128, 16, 4, 1, false>{});
+      return NEXT;
     case 192: fn(RowStepShape<192, 32, 4, 1, false>{}); return true;
     case 256: fn(RowStepShape<256, 32, 4, 1, false>{}); return true;
     case 512: fn(RowStepShape<512, 64, 4, 1, true>{}); return true;
@@ -2533,16 +2539,19 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
   {
     const size_t lds = sizeof(double2) * 3 * padlen(s->H);
     PROF_BEGIN(s, P_ROWS_PRESS);
-    const bool fused_rows = with_row_step(s->H, s->ny, [&](auto S) {
-      using ST = decltype(S);
-      conv = next && fused_cols;
-      auto *kern = s->pressure_on ? (conv ? &k_row_step<ST, true, true> : &k_row_step<ST, true, false>)
-                                  : (conv ? &k_row_step<ST, false, true> : &k_row_step<ST, false, false>);
-      rc = [&]() -> int {
-        KLAUNCH(kern, s->ny / ST::RPB, ST::THREADS, ST::LDS, s->stream, row_step_args(s, mb), s->twx);
-        return FSIBE_OK;
-      }();
-    });
+    auto launch = [&](auto nx) {
+      constexpr bool NEXT = decltype(nx)::value;
+      return with_row_step<NEXT>(s->H, s->ny, [&](auto S) {
+        using ST = decltype(S);
+        auto *kern = s->pressure_on ? &k_row_step<ST, true, NEXT> : &k_row_step<ST, false, NEXT>;
+        rc = [&]() -> int {
+          KLAUNCH(kern, s->ny / ST::RPB, ST::THREADS, ST::LDS, s->stream, row_step_args(s, mb), s->twx);
+          return FSIBE_OK;
+        }();
+      });
+    };
+    conv = next && fused_cols && launch(std::true_type{});
+    const bool fused_rows = conv || launch(std::false_type{});
     CHK(rc);
     if (!fused_rows)
       CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
@@ -3728,7 +3737,7 @@ static void fill_batch_args(fsibe_batch *b, BatchGroup &g, int j, fsibe_sim *s, 
     maxblk[B_K5] = std::max(maxblk[B_K5], a.nblk);
   }
   // K6: the record of the row stage the single path launches
-  const bool rs = with_row_step(s->H, s->ny, [&](auto S) {
+  const bool rs = with_row_step<false>(s->H, s->ny, [&](auto S) {
     RowStepRec &r = reinterpret_cast<RowStepRec *>(A + g.off[B_K6])[j];
     r.a = row_step_args(s, mb);
     r.nblk = s->ny / decltype(S)::RPB;
@@ -3835,7 +3844,7 @@ static int batch_stages(fsibe_batch *b, const std::vector<std::array<int, B_NST>
           break;
         case B_K6: {
           int rc = FSIBE_OK;
-          const bool rs = with_row_step(s0->H, s0->ny, [&](auto S) {
+          const bool rs = with_row_step<false>(s0->H, s0->ny, [&](auto S) {
             using ST = decltype(S);
             auto *kern = g.pres ? &kb_row_step<ST, true, false> : &kb_row_step<ST, false, false>;
             rc = [&]() -> int {
