@@ -25,6 +25,8 @@
 #pragma once
 #include "kernels.hpp"
 
+#include <type_traits>
+
 namespace fsibe {
 
 struct StepConsts {
@@ -53,11 +55,23 @@ constexpr int kCutH = 128;
 
 // entry k of a row of H entries, of which those from kc on are zero and not
 // stored: without a branch around the load (the entries beyond read the last
-// stored one), so that the loads of a row stay in flight together
+// stored one), so that the loads of a row stay in flight together.  CUT false:
+// the caller knows that the row is whole
+template <bool CUT = true>
 __device__ __forceinline__ double2 live(const double2 *__restrict__ row, int k, int H, int kc) {
-  if (H <= kCutH) return row[k];
+  if (!CUT || H <= kCutH) return row[k];
   const double2 v = row[k < kc ? k : kc - 1];
   return k < kc ? v : make_double2(0.0, 0.0);
+}
+
+// fn(cut) for rows of H entries stored up to kc: decided once a row, since the
+// selects cost a whole row some percent of its kernel's time (K2 of the first
+// step of a call, 1024 rows of 512: 18.3 us with them, 17.1 without; 4096 rows
+// 54.5 and 52.3, of 48 with a run-time plan 45.2 and 43.2)
+template <class Fn>
+__device__ __forceinline__ void with_cut(int H, int kc, const Fn &fn) {
+  if (H <= kCutH || kc >= H) fn(std::false_type{});
+  else fn(std::true_type{});
 }
 
 struct MaskBox {
@@ -392,12 +406,15 @@ __device__ __forceinline__ void rows_nl_body(const double2 *__restrict__ A, cons
   const bool prow = penal_on && mb.x1 >= mb.x0 && y >= mb.y0 && y <= mb.y1;
   double ps1 = 0.0, ps2 = 0.0;  // the row's sums of the penalisation term (rowpen)
   // rows: w, dw/dy, dw/dx = i kx w
-  stage_rows_c2r<3>(lds, 3, H, PL, twx, tid, nt, [&](int f, int k) -> double2 {
-    if (f == 1) return live(B + (size_t)y * H, k, H, c.kc);
-    const double2 a = live(A + (size_t)y * H, k, H, c.kc);
-    if (f == 0) return a;
-    const double kf = (double)k * c.sx;
-    return make_double2(-kf * a.y, kf * a.x);
+  with_cut(H, c.kc, [&](auto cut) {
+    constexpr bool CUT = decltype(cut)::value;
+    stage_rows_c2r<3>(lds, 3, H, PL, twx, tid, nt, [&](int f, int k) -> double2 {
+      if (f == 1) return live<CUT>(B + (size_t)y * H, k, H, c.kc);
+      const double2 a = live<CUT>(A + (size_t)y * H, k, H, c.kc);
+      if (f == 0) return a;
+      const double kf = (double)k * c.sx;
+      return make_double2(-kf * a.y, kf * a.x);
+    });
   });
   F.template fft<true, 3>(lds, twx, tid, nt);
   for (int n = tid; n < H; n += nt) {
@@ -635,13 +652,16 @@ __device__ __forceinline__ void rows_press_body(const double2 *__restrict__ Cw, 
   const int nf = mode ? 3 : 2;
   double2 *g1 = mode ? f1 : f0, *g2 = mode ? f2 : f1;  // psi_x, psi_y slots
   // rows: (w,) dpsi/dx = i kx psi, dpsi/dy
-  stage_rows_c2r<3>(lds, nf, H, PL, twx, tid, nt, [&](int f, int k) -> double2 {
-    const int g = mode ? f : f + 1;
-    if (g == 0) return live(Cw + (size_t)y * H, k, H, c.kc);
-    if (g == 2) return live(Cpsiy + (size_t)y * H, k, H, c.kc);
-    const double kf = (double)k * c.sx;
-    const double2 p = live(Cpsi + (size_t)y * H, k, H, c.kc);
-    return make_double2(-kf * p.y, kf * p.x);
+  with_cut(H, c.kc, [&](auto cut) {
+    constexpr bool CUT = decltype(cut)::value;
+    stage_rows_c2r<3>(lds, nf, H, PL, twx, tid, nt, [&](int f, int k) -> double2 {
+      const int g = mode ? f : f + 1;
+      if (g == 0) return live<CUT>(Cw + (size_t)y * H, k, H, c.kc);
+      if (g == 2) return live<CUT>(Cpsiy + (size_t)y * H, k, H, c.kc);
+      const double kf = (double)k * c.sx;
+      const double2 p = live<CUT>(Cpsi + (size_t)y * H, k, H, c.kc);
+      return make_double2(-kf * p.y, kf * p.x);
+    });
   });
   if (mode) F.template fft<true, 3>(lds, twx, tid, nt);
   else F.template fft<true, 2>(lds, twx, tid, nt);
@@ -822,15 +842,18 @@ __device__ __forceinline__ void rows_box_body(const double2 *__restrict__ Cq, co
   const int nf = visc ? 3 : 1;
   // rows: q, and with viscosity d2psi/dxdy = i kx dpsi/dy and
   // d2psi/dy2 - d2psi/dx2 = kx^2 psi + d2psi/dy2
-  stage_rows_c2r<3>(lds, nf, H, PL, twx, tid, nt, [&](int f, int k) -> double2 {
-    if (f == 0) return Cq[(size_t)y * H + k];
-    const double kf = (double)k * c.sx;
-    if (f == 1) {
-      const double2 py = live(Cpsiy + (size_t)y * H, k, H, c.kc);
-      return make_double2(-kf * py.y, kf * py.x);
-    }
-    const double2 p = live(Cpsi + (size_t)y * H, k, H, c.kc), pyy = live(Cpsiyy + (size_t)y * H, k, H, c.kc);
-    return make_double2((kf * kf) * p.x + pyy.x, (kf * kf) * p.y + pyy.y);
+  with_cut(H, c.kc, [&](auto cut) {
+    constexpr bool CUT = decltype(cut)::value;
+    stage_rows_c2r<3>(lds, nf, H, PL, twx, tid, nt, [&](int f, int k) -> double2 {
+      if (f == 0) return Cq[(size_t)y * H + k];
+      const double kf = (double)k * c.sx;
+      if (f == 1) {
+        const double2 py = live<CUT>(Cpsiy + (size_t)y * H, k, H, c.kc);
+        return make_double2(-kf * py.y, kf * py.x);
+      }
+      const double2 p = live<CUT>(Cpsi + (size_t)y * H, k, H, c.kc), pyy = live<CUT>(Cpsiyy + (size_t)y * H, k, H, c.kc);
+      return make_double2((kf * kf) * p.x + pyy.x, (kf * kf) * p.y + pyy.y);
+    });
   });
   if (visc) F.template fft<true, 3>(lds, twx, tid, nt);
   else F.template fft<true, 1>(lds, twx, tid, nt);
