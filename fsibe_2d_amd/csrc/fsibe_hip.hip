@@ -433,7 +433,7 @@ template <class F> struct fixed_len { static constexpr int v = 0; };
 template <int H, int NT> struct fixed_len<RowCT<H, NT>> { static constexpr int v = H; };
 template <int NY, int TX, int NT> struct fixed_len<ColCT<NY, TX, NT>> { static constexpr int v = NY; };
 constexpr bool always_col_step(int ny) { return ny == 128 || ny == 256 || ny == 384 || ny == 512; }
-constexpr bool always_row_step(int H) { return H == 192 || H == 256 || H == 512; }
+constexpr bool always_row_step(int H) { return H == 192 || H == 256; }
 
 // fn(shape) for the fused row stage (K6 and, with NEXT, the convective part of
 // the next K2) of rows of H complex values on ny rows; false if there is none.
@@ -441,8 +441,14 @@ constexpr bool always_row_step(int H) { return H == 192 || H == 256 || H == 512;
 // has no transform then, against K6 alone, us, 256, 1024, 2048 and 4096 rows:
 // 8.3, 11.1, 16.5, 25.4 and 7.3, 9.5, 14.8, 23.6; with the pressure 11.6, 15.2, 20.8,
 // 31.0 and 11.4, 14.5, 20.6, 25.2.
+// Rows of 512 without NEXT: four workgroups of the stage fit a CU, six of K6
+// alone, so that beyond 1024 rows the stage goes in rounds.  Without the
+// pressure (pres) that is slower, with it where the last round is a quarter or
+// less.  Stage and K6 alone at 1024, 1152, 1296, 2048, 2304 and 4096 rows: 15.6, 19.3,
+// 20.2, 27.6, -, 51.9 and 16.3, 17.1, 20.6, 25.9, -, 49.9; with the pressure 20.4, 25.1,
+// 27.4, 36.8, 41.6, 69.7 and 22.6, 23.4, 28.5, 37.6, 39.2, 70.3.
 template <bool NEXT, class Fn>
-static bool with_row_step(int H, int ny, Fn &&fn) {
+static bool with_row_step(int H, int ny, bool pres, Fn &&fn) {
   switch (H) {
     case 32:
       if (ny % 4) return false;
@@ -458,7 +464,10 @@ static bool with_row_step(int H, int ny, Fn &&fn) {
       return NEXT;
     case 192: fn(RowStepShape<192, 32, 4, 1, false>{}); return true;
     case 256: fn(RowStepShape<256, 32, 4, 1, false>{}); return true;
-    case 512: fn(RowStepShape<512, 64, 4, 1, true>{}); return true;
+    case 512:
+      if (!NEXT && ny > 1024 && (!pres || (ny - 1) % 1024 < 256)) return false;
+      fn(RowStepShape<512, 64, 4, 1, true>{});
+      return true;
     default: return false;
   }
 }
@@ -2541,7 +2550,7 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
     PROF_BEGIN(s, P_ROWS_PRESS);
     auto launch = [&](auto nx) {
       constexpr bool NEXT = decltype(nx)::value;
-      return with_row_step<NEXT>(s->H, s->ny, [&](auto S) {
+      return with_row_step<NEXT>(s->H, s->ny, s->pressure_on, [&](auto S) {
         using ST = decltype(S);
         auto *kern = s->pressure_on ? &k_row_step<ST, true, NEXT> : &k_row_step<ST, false, NEXT>;
         rc = [&]() -> int {
@@ -3737,7 +3746,7 @@ static void fill_batch_args(fsibe_batch *b, BatchGroup &g, int j, fsibe_sim *s, 
     maxblk[B_K5] = std::max(maxblk[B_K5], a.nblk);
   }
   // K6: the record of the row stage the single path launches
-  const bool rs = with_row_step<false>(s->H, s->ny, [&](auto S) {
+  const bool rs = with_row_step<false>(s->H, s->ny, g.pres, [&](auto S) {
     RowStepRec &r = reinterpret_cast<RowStepRec *>(A + g.off[B_K6])[j];
     r.a = row_step_args(s, mb);
     r.nblk = s->ny / decltype(S)::RPB;
@@ -3844,7 +3853,7 @@ static int batch_stages(fsibe_batch *b, const std::vector<std::array<int, B_NST>
           break;
         case B_K6: {
           int rc = FSIBE_OK;
-          const bool rs = with_row_step<false>(s0->H, s0->ny, [&](auto S) {
+          const bool rs = with_row_step<false>(s0->H, s0->ny, g.pres, [&](auto S) {
             using ST = decltype(S);
             auto *kern = g.pres ? &kb_row_step<ST, true, false> : &kb_row_step<ST, false, false>;
             rc = [&]() -> int {

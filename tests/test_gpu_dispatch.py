@@ -55,3 +55,45 @@ def test_column_stage_of_long_columns(nx, ny, separate):
         assert np.array_equal(a.field(f), b.field(f)), f
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(1024, 1536), (1024, 2048), (256, 768)])
+@pytest.mark.parametrize("loads", [0, 1])
+def test_row_stage_with_and_without_the_next_term(nx, ny, loads):
+    """rows of 128, and of 512 beyond 1024 of them without the pressure, take
+    the row stage where the next step's term is formed and K6 alone otherwise:
+    the same operations, so the fields, row sums and CFL maximum agree bit for bit"""
+    from fsibe_2d_amd import Params
+    from fsibe_2d_amd.solver import FluidSim
+
+    p = Params(nx=nx, ny=ny, ns=33, nu=2e-3, dt_fixed=1e-4, iSaveBeam=loads, iSponge=0)
+    a, b = FluidSim(p), FluidSim(p)
+    oa = a.run(3)
+    for _ in range(3):
+        ob = b.run(1)
+    for f in ("vortk", "nlk", "u1", "u2", "vor_mean"):
+        assert np.array_equal(a.field(f), b.field(f)), f
+    for k in ("dt1", "u_max", "Force", "energies"):
+        assert oa[k] == ob[k], k
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("nx,ny", [(1024, 1152), (1024, 1296), (1024, 1024)])
+def test_rows_of_512_against_the_oracle(nx, ny, oracle_mod):
+    """K6 alone (1152 rows: a last round of an eighth) and the row stage (1296:
+    more than a quarter; 1024: one round), with the pressure, within the suite's
+    1e-10 of the oracle's fields"""
+    from fsibe_2d_amd import Params
+    from fsibe_2d_amd.solver import FluidSim
+    from tests.conftest import rel_l2
+    from tests.test_gpu_variants import PKEYS
+
+    p = Params(nx=nx, ny=ny, ns=33, nu=2e-3, dt_fixed=1e-4)
+    o = oracle_mod.Oracle(oracle_mod.make_params(**{k: getattr(p, k) for k in PKEYS}))
+    o.run(2)
+    s = FluidSim(p)
+    s.run(2)
+    for k in ("vortk", "u1", "u2", "vor_mean"):
+        assert rel_l2(s.field(k), o.field(k)) <= 1e-10, k
+    s.close()
