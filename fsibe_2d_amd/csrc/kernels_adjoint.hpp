@@ -561,8 +561,9 @@ __device__ __forceinline__ void adj_col_body(const AdjColArgs &a, const double2 
       const double2 lpsi = make_double2(kyf * ya.y + yb.x, -(kyf * ya.x) + yb.y);
       if (!(kx == 0 && ky == 0)) {
         const double quot = (kx2 * c.scalex + ky2 * c.scaley), rq = 1.0 / quot;
-        l.x += div_by(lpsi.x, quot, rq);
-        l.y += div_by(lpsi.y, quot, rq);
+        const double2 d = div_by(lpsi, quot, rq);
+        l.x += d.x;
+        l.y += d.y;
       }
       const double v1 = exp(cx1 * kx2 + cy1 * ky2);
       const double f = v1 * dl[q];

@@ -146,11 +146,18 @@ struct ColStepArgs {
 };
 
 // a / b for a divisor b shared by many quotients, r = 1/b rounded: one
-// Newton correction of a*r rounds as the division does; the fixup takes
-// zeros, infinities and NaN as the division does
-__device__ __forceinline__ double div_by(double a, double b, double r) {
-  const double q = a * r;
-  return __builtin_amdgcn_div_fixup(fma(fma(-q, b, a), r, q), b, a);
+// Newton correction of a*r rounds as the division does while its remainder is
+// exact, and the fixup takes zeros, infinities and NaN as the division does.
+// The remainder of a dividend below 2^-1000 is a denormal number and rounds (up
+// to 5 % of such quotients come out otherwise; a damped mode passes through
+// that range), so dividends below 2^-960 take the division itself.
+__device__ __forceinline__ double2 div_by(double2 a, double b, double r) {
+  const double ax = fabs(a.x), ay = fabs(a.y);
+  if (__builtin_expect((ax < 0x1p-960 && ax != 0.0) || (ay < 0x1p-960 && ay != 0.0), 0))
+    return make_double2(a.x / b, a.y / b);
+  const double qx = a.x * r, qy = a.y * r;
+  return make_double2(__builtin_amdgcn_div_fixup(fma(fma(-qx, b, a.x), r, qx), b, a.x),
+                      __builtin_amdgcn_div_fixup(fma(fma(-qy, b, a.y), r, qy), b, a.y));
 }
 
 // dealias(c, kx, ky) with the divisions left to the modes on the ellipse's
@@ -281,7 +288,7 @@ __device__ __forceinline__ void col_step_body(const ColStepArgs &a, const double
           }
           if (kx != 0 || ky != 0) {
             const double quot = kx2 * c.scalex + ky2 * c.scaley, rq = 1.0 / quot;
-            psi = make_double2(div_by(w1.x, quot, rq), div_by(w1.y, quot, rq));
+            psi = div_by(w1, quot, rq);
           }
         }
         const size_t g = (size_t)idx * H + kx;
@@ -421,7 +428,7 @@ __device__ __forceinline__ void col_direct_body(const ColStepArgs &a, const doub
         const int idx = t + NT * q, ky = ky_signed(idx, L), aky = ky < 0 ? -ky : ky;
         if (idx != L / 2 && (kx != 0 || ky != 0)) {
           const double quot = (double)(kx * kx) * c.scalex + (double)(aky * aky) * c.scaley, rq = 1.0 / quot;
-          W[q] = make_double2(div_by(W[q].x, quot, rq), div_by(W[q].y, quot, rq));
+          W[q] = div_by(W[q], quot, rq);
         } else {
           W[q] = make_double2(0.0, 0.0);
         }
@@ -494,7 +501,7 @@ __device__ __forceinline__ double2 press_mode(const StepConsts &c, int kx, int i
   const double2 fb = make_double2(b.x * c.norm, b.y * c.norm);
   const double2 rhs = make_double2(fa.x - kyf * fb.y, fa.y + kyf * fb.x);
   const double quot = ((double)(kx * kx) * c.scalex + (double)(aky * aky) * c.scaley), rq = 1.0 / quot;
-  return make_double2(div_by(rhs.x, quot, rq), div_by(rhs.y, quot, rq));
+  return div_by(rhs, quot, rq);
 }
 
 // Two slots of TX*NT threads transform one right-hand side each straight from
@@ -699,7 +706,8 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
     um = fmax(um, fmax(a1.x * a1.x + a2.x * a2.x, a1.y * a1.y + a2.y * a2.y));
     {
       const double2 v = vm[k];
-      reinterpret_cast<double2 *>(a.vor_mean + rowx)[n] = make_double2(div_by(v.x * time + dt1 * w.x, tsum, trcp), div_by(v.y * time + dt1 * w.y, tsum, trcp));
+      reinterpret_cast<double2 *>(a.vor_mean + rowx)[n] =
+          div_by(make_double2(v.x * time + dt1 * w.x, v.y * time + dt1 * w.y), tsum, trcp);
     }
     en[0] += w.x * w.x + w.y * w.y;
     {
