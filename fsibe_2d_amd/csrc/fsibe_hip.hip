@@ -439,11 +439,12 @@ constexpr bool always_row_step(int H) { return H == 192 || H == 256; }
 // the next K2) of rows of H complex values on ny rows; false if there is none.
 // Rows of 128 without NEXT: the stage's one wave a row, of which a quarter
 // has no transform then, against K6 alone, us, 256, 1024, 2048 and 4096 rows:
-// 8.3, 11.1, 16.5, 25.4 and 7.3, 9.5, 14.8, 23.6; with the pressure 11.6, 15.2, 20.8,
-// 31.0 and 11.4, 14.5, 20.6, 25.2.
+// 8.3, 11.1, 16.5, 25.4 and 7.3, 9.5, 14.8, 23.6; with the pressure (pres) 11.6, 15.2,
+// 20.8, 31.0 and 11.4, 14.5, 20.6, 25.2, where only the last makes a difference
+// to a step (a coupled 256^2 step is 0.6 % faster with the stage).
 // Rows of 512 without NEXT: four workgroups of the stage fit a CU, six of K6
 // alone, so that beyond 1024 rows the stage goes in rounds.  Without the
-// pressure (pres) that is slower, with it where the last round is a quarter or
+// pressure that is slower, with it where the last round is a quarter or
 // less.  Stage and K6 alone at 1024, 1152, 1296, 2048, 2304 and 4096 rows: 15.6, 19.3,
 // 20.2, 27.6, -, 51.9 and 16.3, 17.1, 20.6, 25.9, -, 49.9; with the pressure 20.4, 25.1,
 // 27.4, 36.8, 41.6, 69.7 and 22.6, 23.4, 28.5, 37.6, 39.2, 70.3.
@@ -460,8 +461,9 @@ static bool with_row_step(int H, int ny, bool pres, Fn &&fn) {
       return true;
     case 96: fn(RowStepShape<96, 16, 4, 1, false>{}); return true;
     case 128:
-      if constexpr (NEXT) fn(RowStepShape<128, 16, 4, 1, false>{});
-      return NEXT;
+      if (!NEXT && (!pres || ny > 2048)) return false;
+      fn(RowStepShape<128, 16, 4, 1, false>{});
+      return true;
     case 192: fn(RowStepShape<192, 32, 4, 1, false>{}); return true;
     case 256: fn(RowStepShape<256, 32, 4, 1, false>{}); return true;
     case 512:
