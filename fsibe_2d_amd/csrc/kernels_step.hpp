@@ -842,18 +842,15 @@ __device__ __forceinline__ void rows_box_body(const double2 *__restrict__ Cq, co
   const int nf = visc ? 3 : 1;
   // rows: q, and with viscosity d2psi/dxdy = i kx dpsi/dy and
   // d2psi/dy2 - d2psi/dx2 = kx^2 psi + d2psi/dy2
-  with_cut(H, c.kc, [&](auto cut) {
-    constexpr bool CUT = decltype(cut)::value;
-    stage_rows_c2r<3>(lds, nf, H, PL, twx, tid, nt, [&](int f, int k) -> double2 {
-      if (f == 0) return Cq[(size_t)y * H + k];
-      const double kf = (double)k * c.sx;
-      if (f == 1) {
-        const double2 py = live<CUT>(Cpsiy + (size_t)y * H, k, H, c.kc);
-        return make_double2(-kf * py.y, kf * py.x);
-      }
-      const double2 p = live<CUT>(Cpsi + (size_t)y * H, k, H, c.kc), pyy = live<CUT>(Cpsiyy + (size_t)y * H, k, H, c.kc);
-      return make_double2((kf * kf) * p.x + pyy.x, (kf * kf) * p.y + pyy.y);
-    });
+  stage_rows_c2r<3>(lds, nf, H, PL, twx, tid, nt, [&](int f, int k) -> double2 {
+    if (f == 0) return Cq[(size_t)y * H + k];
+    const double kf = (double)k * c.sx;
+    if (f == 1) {
+      const double2 py = live(Cpsiy + (size_t)y * H, k, H, c.kc);
+      return make_double2(-kf * py.y, kf * py.x);
+    }
+    const double2 p = live(Cpsi + (size_t)y * H, k, H, c.kc), pyy = live(Cpsiyy + (size_t)y * H, k, H, c.kc);
+    return make_double2((kf * kf) * p.x + pyy.x, (kf * kf) * p.y + pyy.y);
   });
   if (visc) F.template fft<true, 3>(lds, twx, tid, nt);
   else F.template fft<true, 1>(lds, twx, tid, nt);
