@@ -440,35 +440,37 @@ constexpr bool always_row_step(int H) { return H == 192 || H == 256; }
 // Rows of 128 without NEXT: the stage's one wave a row, of which a quarter
 // has no transform then, against K6 alone, us, 256, 1024, 2048 and 4096 rows:
 // 8.3, 11.1, 16.5, 25.4 and 7.3, 9.5, 14.8, 23.6; with the pressure (pres) 11.6, 15.2,
-// 20.8, 31.0 and 11.4, 14.5, 20.6, 25.2, where only the last makes a difference
-// to a step (a coupled 256^2 step is 0.6 % faster with the stage).
+// 20.8, 31.0 and 11.4, 14.5, 20.6, 25.2, where only the last shows in a step.
 // Rows of 512 without NEXT: four workgroups of the stage fit a CU, six of K6
 // alone, so that beyond 1024 rows the stage goes in rounds.  Without the
 // pressure that is slower, with it where the last round is a quarter or
 // less.  Stage and K6 alone at 1024, 1152, 1296, 2048, 2304 and 4096 rows: 15.6, 19.3,
 // 20.2, 27.6, -, 51.9 and 16.3, 17.1, 20.6, 25.9, -, 49.9; with the pressure 20.4, 25.1,
 // 27.4, 36.8, 41.6, 69.7 and 22.6, 23.4, 28.5, 37.6, 39.2, 70.3.
+// Lengths without a shape: 384, 37 us against 30 of K6 and K2 at 768 x 768; 1024
+// and more, whose four buffers leave one or two rows on a CU (2048^2: 112 to 200 us
+// in the shapes tried, K6 80 and K2 54); 48, 768 and lengths with a 9: not tried.
 template <bool NEXT, class Fn>
 static bool with_row_step(int H, int ny, bool pres, Fn &&fn) {
   switch (H) {
     case 32:
       if (ny % 4) return false;
-      fn(RowStepShape<32, 4, 4, 4, false>{});
+      fn(RowStepShape<32, 4, 4, false>{});
       return true;
     case 64:
       if (ny % 2) return false;
-      fn(RowStepShape<64, 8, 4, 2, false>{});
+      fn(RowStepShape<64, 8, 2, false>{});
       return true;
-    case 96: fn(RowStepShape<96, 16, 4, 1, false>{}); return true;
+    case 96: fn(RowStepShape<96, 16, 1, false>{}); return true;
     case 128:
       if (!NEXT && (!pres || ny > 2048)) return false;
-      fn(RowStepShape<128, 16, 4, 1, false>{});
+      fn(RowStepShape<128, 16, 1, false>{});
       return true;
-    case 192: fn(RowStepShape<192, 32, 4, 1, false>{}); return true;
-    case 256: fn(RowStepShape<256, 32, 4, 1, false>{}); return true;
+    case 192: fn(RowStepShape<192, 32, 1, false>{}); return true;
+    case 256: fn(RowStepShape<256, 32, 1, false>{}); return true;
     case 512:
       if (!NEXT && ny > 1024 && (!pres || (ny - 1) % 1024 < 256)) return false;
-      fn(RowStepShape<512, 64, 4, 1, true>{});
+      fn(RowStepShape<512, 64, 1, true>{});
       return true;
     default: return false;
   }
@@ -533,10 +535,9 @@ extern "C" int fsibe_spectral_destroy(fsibe_spectral *c) {
   return FSIBE_OK;
 }
 
-// real rows -> half spectrum (unnormalised)
 // fn(shape) for row transforms of H complex values; false if there is none.
-// Threads and rows per workgroup as measured (kernels_spectral.hpp): about H/8
-// threads a row, more where that leaves the last pass uneven.
+// Threads and rows per workgroup are the fastest measured: H/4 threads a row up
+// to 256 values and H/8 from 512 on, H/3 or H/6 where the length holds a 3.
 template <class Fn>
 static bool with_rows_io(int H, Fn &&fn) {
   switch (H) {
@@ -581,8 +582,8 @@ static bool with_cols_io(int ny, int H, Fn &&fn) {
   }
 }
 
-// fn(shape) for a grid of up to 2048 half-spectrum entries in one workgroup;
-// false if there is none
+// fn(shape) for a grid in one workgroup, 64 x 64, 128 x 32 and 64 x 32; false for
+// the others (twice the entries gain nothing: kernels_spectral.hpp)
 template <class Fn>
 static bool with_small(int H, int ny, Fn &&fn) {
   if (H == 32 && ny == 64) { fn(SmallShape<32, 64, 4, 8, 512>{}); return true; }
@@ -591,6 +592,7 @@ static bool with_small(int H, int ny, Fn &&fn) {
   return false;
 }
 
+// real rows -> half spectrum (unnormalised)
 static int rows_r2c(int nx, int ny, const FftPlan &px, const double2 *twx, const double *f, double2 *out,
                     hipStream_t st) {
   int rc = FSIBE_OK;
@@ -3863,7 +3865,7 @@ static int batch_stages(fsibe_batch *b, const std::vector<std::array<int, B_NST>
           int rc = FSIBE_OK;
           const bool rs = with_row_step<false>(s0->H, s0->ny, g.pres, [&](auto S) {
             using ST = decltype(S);
-            auto *kern = g.pres ? &kb_row_step<ST, true, false> : &kb_row_step<ST, false, false>;
+            auto *kern = g.pres ? &kb_row_step<ST, true> : &kb_row_step<ST, false>;
             rc = [&]() -> int {
               SLAUNCH(kern, gx, nm, ST::THREADS, ST::LDS, g.stream, mode,
                       reinterpret_cast<const RowStepRec *>(arr(g, B_K6)), s0->twx);

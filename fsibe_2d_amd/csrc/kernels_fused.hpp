@@ -467,17 +467,6 @@ template <class S>
 __global__ void __launch_bounds__(S::THREADS) k_col_step(ColStepArgs a, const double2 *__restrict__ twy) {
   S::run(a, twy, blockIdx.x, gridDim.x);
 }
-struct ColStepRec {
-  ColStepArgs a;
-  int nblk, pad;
-};
-template <class S>
-__global__ void __launch_bounds__(S::THREADS) kb_col_step(const ColStepRec *__restrict__ arr,
-                                                          const double2 *__restrict__ twy) {
-  const ColStepRec &r = arr[blockIdx.y];
-  if ((int)blockIdx.x >= r.nblk) return;
-  S::run(r.a, twy, blockIdx.x, r.nblk);
-}
 
 // ============================================================================
 // Pressure stage (K7)
@@ -605,20 +594,19 @@ __device__ __forceinline__ double2 c2r_elem(double2 xa, double2 xq, int e, doubl
 }
 __device__ __forceinline__ double2 mul_ik(double2 a, double kf) { return make_double2(-kf * a.y, kf * a.x); }
 
-// One row by NS slots of NT threads, RPB rows per workgroup.  Inverse
+// One row by four slots of NT threads, RPB rows per workgroup.  Inverse
 // transforms of psi_y, psi_x, omega and (NEXT) omega_x, one per slot; then
 // velocity, diagnostics and products; forward transforms of the pressure
 // right-hand sides (PRES) beside the inverse one of omega_y (in slot 2, as
 // the conjugate of a forward transform of the conjugate: the same
-// operations); then the convective term's forward transform.  With a fifth
-// slot omega_y goes with the first four.
-template <int H, int NT, int NS, int RPB, bool LEAN, bool PRES, bool NEXT>
+// operations); then the convective term's forward transform.
+template <int H, int NT, int RPB, bool LEAN, bool PRES, bool NEXT>
 __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double2 *__restrict__ twx, int bid) {
   extern __shared__ double2 lds[];
-  constexpr int PL = padlen(H), nx = 2 * H, NR = NS * NT;  // NR threads per row
-  constexpr bool WAVE = NR <= 64, FIVE = NS == 5;
+  constexpr int NS = 4, PL = padlen(H), nx = 2 * H, NR = NS * NT;  // NR threads per row
+  constexpr bool WAVE = NR <= 64;
   constexpr int PN = (H + NR - 1) / NR;
-  static_assert(NS >= (NEXT ? 4 : 3) && NS <= 5 && (!WAVE || (NR & (NR - 1)) == 0), "slots");
+  static_assert(!WAVE || (NR & (NR - 1)) == 0, "slots");
   static_assert(RPB == 1 || (WAVE && 64 % NR == 0), "several rows per workgroup: each within one wave");
   using Out = FftOut<H, NT>;
   const int tid = threadIdx.x, rr = RPB == 1 ? 0 : tid / NR, p = RPB == 1 ? tid : tid - rr * NR;
@@ -662,7 +650,7 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
   }
   double2 z[Out::N];
   {
-    const double2 *src = slot == 0 ? a.Cpsiy : slot == 1 ? a.Cpsi : (FIVE && slot == 4) ? a.Cwy : a.Cw;
+    const double2 *src = slot == 0 ? a.Cpsiy : slot == 1 ? a.Cpsi : a.Cw;
     const bool ik = slot == 1 || slot == 3;
     src += rowk;
     const int kc = a.c.kc;
@@ -687,7 +675,7 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
   const bool wrow2 = two && y >= win2.y0 && y <= win2.y1;
   const double tsum = time + dt1, trcp = 1.0 / tsum;
   double um = 0.0, en[2] = {0.0, 0.0};
-  double2 csw[NEXT && !FIVE ? PN : 1];
+  double2 csw[NEXT ? PN : 1];
 #pragma unroll
   for (int k = 0; k < PN; ++k) {
     const int n = p + k * NR;
@@ -719,13 +707,8 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
       const double2 s = ms[k];
       const double2 cv = make_double2(-(a1.x * wx.x), -(a1.y * wx.y));
       const double2 sw = make_double2(s.x * w.x, s.y * w.y);
-      if constexpr (FIVE) {
-        const double2 wy = row[4 * PL + qn];
-        row[3 * PL + qn] = make_double2((cv.x - a2.x * wy.x) - sw.x, (cv.y - a2.y * wy.y) - sw.y);
-      } else {
-        row[3 * PL + qn] = cv;  // this thread takes it back below
-        csw[k] = sw;
-      }
+      row[3 * PL + qn] = cv;  // this thread takes it back below
+      csw[k] = sw;
     }
     // penal(:,:,1) - vor*uy, penal(:,:,2) + vor*ux (:357-358); on the mask's
     // rows the velocity is left for the loop below, which adds the
@@ -838,11 +821,10 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
   using One = std::integral_constant<int, 1>;
   using Two = std::integral_constant<int, 2>;
   // second round: forward transforms of the pressure right-hand sides (slots
-  // 0, 1), and slot 2 the inverse of omega_y (or, with five slots,
-  // slot 3 the forward one of the convective term)
+  // 0, 1), and slot 2 the inverse of omega_y
   {
-    const bool inv = NEXT && !FIVE && slot == 2;
-    const bool act = (PRES && slot < 2) || (NEXT && slot == (FIVE ? 3 : 2));
+    const bool inv = NEXT && slot == 2;
+    const bool act = (PRES && slot < 2) || inv;
     double2 in[NI];
     if constexpr (LEAN) asm volatile("" : "+v"(t));
     if (inv) {
@@ -866,8 +848,7 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
       a.Rq[rowk + k] = mul_ik(x[0], (double)k * sx);
       a.Rqy[rowk + k] = x[1];
     });
-  if constexpr (NEXT && FIVE) post(One{}, 3, [&](int k, const double2 *x) { a.Rc[rowk + k] = x[0]; });
-  if constexpr (NEXT && !FIVE) {
+  if constexpr (NEXT) {
 #pragma unroll
     for (int k = 0; k < PN; ++k) {
       const int n = p + k * NR;
@@ -888,8 +869,8 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
   }
 }
 
-template <int HC, int NTC, int NSC, int RPBC, bool LEANC> struct RowStepShape {
-  static constexpr int H = HC, NT = NTC, NS = NSC, RPB = RPBC;
+template <int HC, int NTC, int RPBC, bool LEANC> struct RowStepShape {
+  static constexpr int H = HC, NT = NTC, NS = 4, RPB = RPBC;
   static constexpr bool LEAN = LEANC;
   static constexpr int THREADS = NS * NT * RPB;
   static constexpr size_t LDS = sizeof(double2) * NS * padlen(H) * RPB;
@@ -899,18 +880,18 @@ template <int HC, int NTC, int NSC, int RPBC, bool LEANC> struct RowStepShape {
 template <class S, bool PRES, bool NEXT>
 __global__ void __launch_bounds__(S::THREADS) __attribute__((amdgpu_waves_per_eu(S::LEAN ? 4 : 1, 8)))
 k_row_step(RowStepArgs a, const double2 *__restrict__ twx) {
-  row_step_body<S::H, S::NT, S::NS, S::RPB, S::LEAN, PRES, NEXT>(a, twx, blockIdx.x);
+  row_step_body<S::H, S::NT, S::RPB, S::LEAN, PRES, NEXT>(a, twx, blockIdx.x);
 }
 struct RowStepRec {
   RowStepArgs a;
   int nblk, pad;
 };
-template <class S, bool PRES, bool NEXT>
+template <class S, bool PRES>
 __global__ void __launch_bounds__(S::THREADS) __attribute__((amdgpu_waves_per_eu(S::LEAN ? 4 : 1, 8)))
 kb_row_step(const RowStepRec *__restrict__ arr, const double2 *__restrict__ twx) {
   const RowStepRec &r = arr[blockIdx.y];
   if ((int)blockIdx.x >= r.nblk) return;
-  row_step_body<S::H, S::NT, S::NS, S::RPB, S::LEAN, PRES, NEXT>(r.a, twx, blockIdx.x);
+  row_step_body<S::H, S::NT, S::RPB, S::LEAN, PRES, false>(r.a, twx, blockIdx.x);
 }
 
 }  // namespace fsibe

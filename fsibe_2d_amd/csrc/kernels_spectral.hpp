@@ -7,9 +7,9 @@
 // kernel reads and writes the field once).  Against the kernels that stage
 // their rows or columns in LDS first, forward and backward together: 256^2
 // 16.5 -> 14.4 us, 384^2 19.8 -> 17.2, 512^2 21.8 -> 17.1, 1024^2 37.5 -> 31.2,
-// 2048^2 70.9 -> 64.6.  Grids of up to 2048 half-spectrum entries take one
-// workgroup and one kernel for both directions: 64^2 forward 5.7 -> 4.4 us,
-// backward 5.6 -> 4.0 (128 x 64, with twice the entries: 5.9 -> 5.7, not taken).
+// 2048^2 70.9 -> 64.6.  Grids of 64 x 64, 128 x 32 and 64 x 32 take one
+// workgroup and one kernel a direction: 64^2 forward 5.7 -> 4.4 us, backward 5.6
+// -> 4.0 (128 x 64, with twice the entries: 5.9 -> 5.7, not taken).
 // The same passes and formulas as those kernels, so the same bits.
 #pragma once
 #include "kernels_fused.hpp"

@@ -67,7 +67,7 @@ __device__ __forceinline__ double2 live(const double2 *__restrict__ row, int k, 
 // fn(cut) for rows of H entries stored up to kc: decided once a row, since the
 // selects cost a whole row some percent of its kernel's time (K2 of the first
 // step of a call, 1024 rows of 512: 18.3 us with them, 17.1 without; 4096 rows
-// 54.5 and 52.3, of 48 with a run-time plan 45.2 and 43.2)
+// 54.5 and 52.3)
 template <class Fn>
 __device__ __forceinline__ void with_cut(int H, int kc, const Fn &fn) {
   if (H <= kCutH || kc >= H) fn(std::false_type{});
