@@ -150,14 +150,21 @@ struct ColStepArgs {
 // exact, and the fixup takes zeros, infinities and NaN as the division does.
 // The remainder of a dividend below 2^-1000 is a denormal number and rounds (up
 // to 5 % of such quotients come out otherwise; a damped mode passes through
-// that range), so dividends below 2^-960 take the division itself.
-__device__ __forceinline__ double2 div_by(double2 a, double b, double r) {
-  const double ax = fabs(a.x), ay = fabs(a.y);
-  if (__builtin_expect((ax < 0x1p-960 && ax != 0.0) || (ay < 0x1p-960 && ay != 0.0), 0))
-    return make_double2(a.x / b, a.y / b);
+// that range), so where a wave meets a dividend below 2^-960 (div_small) it
+// divides.  The choice is made once for all of a thread's quotients: a branch
+// at each cost a coupled 256^2 step 0.7 % and two beams at 768 x 512 1 %.
+__device__ __forceinline__ double2 div_fast(double2 a, double b, double r) {
   const double qx = a.x * r, qy = a.y * r;
   return make_double2(__builtin_amdgcn_div_fixup(fma(fma(-qx, b, a.x), r, qx), b, a.x),
                       __builtin_amdgcn_div_fixup(fma(fma(-qy, b, a.y), r, qy), b, a.y));
+}
+__device__ __forceinline__ bool div_small(double2 a) {
+  const double x = fabs(a.x), y = fabs(a.y);
+  return (x < 0x1p-960 && x != 0.0) || (y < 0x1p-960 && y != 0.0);
+}
+__device__ __forceinline__ double2 div_slow(double2 a, double b) { return make_double2(a.x / b, a.y / b); }
+__device__ __forceinline__ double2 div_by(double2 a, double b, double r) {
+  return __builtin_expect(div_small(a), 0) ? div_slow(a, b) : div_fast(a, b, r);
 }
 
 // dealias(c, kx, ky) with the divisions left to the modes on the ellipse's
@@ -255,6 +262,7 @@ __device__ __forceinline__ void col_step_body(const ColStepArgs &a, const double
     // a constant time step: both viscous factors are the same number
     const bool same = cx0 == cx1 && cy0 == cy1;
     const double kx2 = (double)(kx * kx);
+    bool small = false;
     if constexpr (!PREF) {
 #pragma unroll
       for (int q = 0; q < EL; ++q) operands(q);
@@ -288,7 +296,8 @@ __device__ __forceinline__ void col_step_body(const ColStepArgs &a, const double
           }
           if (kx != 0 || ky != 0) {
             const double quot = kx2 * c.scalex + ky2 * c.scaley, rq = 1.0 / quot;
-            psi = div_by(w1, quot, rq);
+            psi = div_fast(w1, quot, rq);
+            small = small || div_small(w1);
           }
         }
         const size_t g = (size_t)idx * H + kx;
@@ -296,6 +305,14 @@ __device__ __forceinline__ void col_step_body(const ColStepArgs &a, const double
         a.W1[g] = w1;
         w0[q] = w1;
         n1[q] = psi;
+      }
+    }
+    if (__builtin_expect(__any(small), 0)) {
+#pragma unroll
+      for (int q = 0; q < EL; ++q) {
+        const int idx = i0 + q * (NTHR / TX), ky = ky_signed(idx, L);
+        if (idx != L / 2 && (kx != 0 || ky != 0))
+          n1[q] = div_slow(w0[q], kx2 * c.scalex + (double)(ky * ky) * c.scaley);
       }
     }
   }
@@ -422,17 +439,25 @@ __device__ __forceinline__ void col_direct_body(const ColStepArgs &a, const doub
     const int f = kF[k];
     double2 *out = a.o[f];
     if (k == 2) {
+      bool small = false;
 #pragma unroll
-      for (int q = 0; q < E; ++q) {
-        if (q % 2 == 0) __builtin_amdgcn_sched_barrier(0);
-        const int idx = t + NT * q, ky = ky_signed(idx, L), aky = ky < 0 ? -ky : ky;
-        if (idx != L / 2 && (kx != 0 || ky != 0)) {
-          const double quot = (double)(kx * kx) * c.scalex + (double)(aky * aky) * c.scaley, rq = 1.0 / quot;
-          W[q] = div_by(W[q], quot, rq);
-        } else {
-          W[q] = make_double2(0.0, 0.0);
+      for (int q = 0; q < E; ++q) small = small || div_small(W[q]);
+      auto psi = [&](auto slow) {
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+          if (q % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+          const int idx = t + NT * q, ky = ky_signed(idx, L), aky = ky < 0 ? -ky : ky;
+          if (idx != L / 2 && (kx != 0 || ky != 0)) {
+            const double quot = (double)(kx * kx) * c.scalex + (double)(aky * aky) * c.scaley;
+            if constexpr (decltype(slow)::value) W[q] = div_slow(W[q], quot);
+            else W[q] = div_fast(W[q], quot, 1.0 / quot);
+          } else {
+            W[q] = make_double2(0.0, 0.0);
+          }
         }
-      }
+      };
+      if (__builtin_expect(__any(small), 0)) psi(std::true_type{});
+      else psi(std::false_type{});
     }
     if (!out) continue;
     const int ya = f == 3 ? a.r0 : 0, yb = f == 3 ? a.r1 : L - 1;
@@ -478,19 +503,20 @@ struct PressArgs {
   StepConsts c;
 };
 
-// the spectrum of q at mode (kx, idx) from the transforms of the two
-// right-hand sides (pressure, NavierStokes.f90:366-382)
+// the right-hand side of q's equation at mode (kx, idx) from the transforms of
+// its two parts (pressure, NavierStokes.f90:366-382), and |k|^2 in quot (1 at the
+// modes that are zero)
 template <int L>
-__device__ __forceinline__ double2 press_mode(const StepConsts &c, int kx, int idx, double2 a, double2 b) {
+__device__ __forceinline__ double2 press_rhs(const StepConsts &c, int kx, int idx, double2 a, double2 b, double &quot) {
   const int ky = ky_signed(idx, L);
   const int aky = ky < 0 ? -ky : ky;
+  quot = 1.0;
   if (idx == L / 2 || (kx == 0 && ky == 0)) return make_double2(0.0, 0.0);
   const double kyf = (double)ky * c.sy;
   const double2 fa = make_double2(a.x * c.norm, a.y * c.norm);
   const double2 fb = make_double2(b.x * c.norm, b.y * c.norm);
-  const double2 rhs = make_double2(fa.x - kyf * fb.y, fa.y + kyf * fb.x);
-  const double quot = ((double)(kx * kx) * c.scalex + (double)(aky * aky) * c.scaley), rq = 1.0 / quot;
-  return div_by(rhs, quot, rq);
+  quot = ((double)(kx * kx) * c.scalex + (double)(aky * aky) * c.scaley);
+  return make_double2(fa.x - kyf * fb.y, fa.y + kyf * fb.x);
 }
 
 // Two slots of TX*NT threads transform one right-hand side each straight from
@@ -530,10 +556,26 @@ __device__ __forceinline__ void press_step_body(const PressArgs &a, const double
     }
     grp_sync<WAVE>();
   }
-  for (int e = tid; e < L * TX; e += NTHR) {
-    const int idx = e / TX, c2 = e % TX;
-    double2 *l0 = lds + pidx(idx) * TX + c2;
-    *l0 = press_mode<L>(c, kx0 + c2, idx, l0[0], l0[SB]);
+  {
+    constexpr int EL = L * TX / NTHR;
+    static_assert(L * TX % NTHR == 0, "every thread has as many modes");
+    double2 rhs[EL];
+    double quot[EL];
+    bool small = false;
+    auto at = [&](int q) { return lds + pidx((tid + q * NTHR) / TX) * TX + (tid + q * NTHR) % TX; };
+#pragma unroll
+    for (int q = 0; q < EL; ++q) {
+      const int e = tid + q * NTHR;
+      rhs[q] = press_rhs<L>(c, kx0 + e % TX, e / TX, at(q)[0], at(q)[SB], quot[q]);
+      small = small || div_small(rhs[q]);
+    }
+    if (__builtin_expect(__any(small), 0)) {
+#pragma unroll
+      for (int q = 0; q < EL; ++q) *at(q) = div_slow(rhs[q], quot[q]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < EL; ++q) *at(q) = div_fast(rhs[q], quot[q], 1.0 / quot[q]);
+    }
   }
   grp_sync<WAVE>();
   fft_io<L, NT, true, TX, WAVE, false>(
@@ -675,6 +717,7 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
   const bool wrow2 = two && y >= win2.y0 && y <= win2.y1;
   const double tsum = time + dt1, trcp = 1.0 / tsum;
   double um = 0.0, en[2] = {0.0, 0.0};
+  bool small = false;
   double2 csw[NEXT ? PN : 1];
 #pragma unroll
   for (int k = 0; k < PN; ++k) {
@@ -693,9 +736,9 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
     reinterpret_cast<double2 *>(a.u2 + rowx)[n] = a2;
     um = fmax(um, fmax(a1.x * a1.x + a2.x * a2.x, a1.y * a1.y + a2.y * a2.y));
     {
-      const double2 v = vm[k];
-      reinterpret_cast<double2 *>(a.vor_mean + rowx)[n] =
-          div_by(make_double2(v.x * time + dt1 * w.x, v.y * time + dt1 * w.y), tsum, trcp);
+      const double2 m = make_double2(vm[k].x * time + dt1 * w.x, vm[k].y * time + dt1 * w.y);
+      reinterpret_cast<double2 *>(a.vor_mean + rowx)[n] = div_fast(m, tsum, trcp);
+      small = small || div_small(m);
     }
     en[0] += w.x * w.x + w.y * w.y;
     {
@@ -719,6 +762,16 @@ __device__ __forceinline__ void row_step_body(const RowStepArgs &a, const double
     } else if (PRES) {
       row[qn] = make_double2(0.0 - w.x * a2.x, 0.0 - w.y * a2.y);
       row[PL + qn] = make_double2(0.0 + w.x * a1.x, 0.0 + w.y * a1.y);
+    }
+  }
+  if (__builtin_expect(__any(small), 0)) {
+#pragma unroll
+    for (int k = 0; k < PN; ++k) {
+      const int n = p + k * NR;
+      if (H % NR != 0 && n >= H) continue;
+      const double2 w = row[2 * PL + pidx(n)];
+      reinterpret_cast<double2 *>(a.vor_mean + rowx)[n] =
+          div_slow(make_double2(vm[k].x * time + dt1 * w.x, vm[k].y * time + dt1 * w.y), tsum);
     }
   }
   // the mask's rows: penalisation p = chi (u - u_s), its sums, and the
