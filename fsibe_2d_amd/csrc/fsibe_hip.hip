@@ -2366,6 +2366,16 @@ static int launch_k1(fsibe_sim *s, int level, bool have_a = false) {
   return FSIBE_OK;
 }
 
+// K2's instance for rows by F: rows of at most kCutH entries are never cut, longer
+// ones whole only on a call's first step or without dealiasing, where the selects
+// cost little of the call with a compile-time plan (1024 rows of 512: 18.3 us and
+// 17.1 without) and 2 % of a step with a run-time one
+template <class F> static auto nl_kernel(const fsibe_sim *s) {
+  constexpr int H = fixed_len<F>::v;
+  if constexpr (H > 0) return &k_rows_nl<F, (H > kCutH)>;
+  else return s->kcA < s->H ? &k_rows_nl<F, true> : &k_rows_nl<F, false>;
+}
+
 // the constants of K2: columns of A, B beyond kcA are zero and not stored
 static StepConsts nl_consts(const fsibe_sim *s) {
   StepConsts c = s->sc;
@@ -2387,7 +2397,8 @@ static int launch_k2_ahead(fsibe_sim *s) {
   none.m = none.vx = none.vy = nullptr;
   const size_t lds = sizeof(double2) * 3 * padlen(s->H);
   CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
-    KLAUNCH(k_rows_nl<decltype(F)>, na + nb, nt, lds, s->stream, s->T[0], s->Bp, s->u1, s->u2,
+    auto *kern = nl_kernel<decltype(F)>(s);
+    KLAUNCH(kern, na + nb, nt, lds, s->stream, s->T[0], s->Bp, s->u1, s->u2,
             s->sponge_on ? s->ms : nullptr, none, (int)s->penal_on, s->T[2], s->penal_on ? s->T[3] : nullptr,
             F, s->twx, nl_consts(s),
             s->umax_part, s->ny, s->dscal, s->fp, 0.0, 0.0, 0, res_dev(s, s->slot), 0, na, b1 + 1, 0,
@@ -2475,7 +2486,8 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
       // ev_dt at K2's end: the host reads dt1 and then the previous step's
       // results (kernels before this one in the stream)
       CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
-        KLAUNCH_EV(k_rows_nl<decltype(F)>, s->ny, nt, lds, s->stream, s->ev_dt, s->T[0], s->Bp, s->u1, s->u2,
+        auto *kern = nl_kernel<decltype(F)>(s);
+        KLAUNCH_EV(kern, s->ny, nt, lds, s->stream, s->ev_dt, s->T[0], s->Bp, s->u1, s->u2,
                    s->sponge_on ? s->ms : nullptr, mb, (int)s->penal_on, s->T[2], s->penal_on ? s->T[3] : nullptr,
                    F, s->twx, nl_consts(s),
                    s->umax_part, s->ny, s->dscal, s->fp, time, dt0, (int)explicit_step, res_dev(s, s->slot), 0,
@@ -2484,7 +2496,8 @@ static int evolve_fluid(fsibe_sim *s, double time, double dt0, bool explicit_ste
       }));
     } else {
       CHK(with_rows<3>(s->px, [&](auto F, int nt) -> int {
-        KLAUNCH(k_rows_nl<decltype(F)>, s->ny, nt, lds, s->stream, s->T[0], s->Bp, s->u1, s->u2,
+        auto *kern = nl_kernel<decltype(F)>(s);
+        KLAUNCH(kern, s->ny, nt, lds, s->stream, s->T[0], s->Bp, s->u1, s->u2,
                 s->sponge_on ? s->ms : nullptr, mb, (int)s->penal_on, s->T[2], s->penal_on ? s->T[3] : nullptr,
                 F, s->twx, nl_consts(s),
                 s->umax_part, s->ny, s->dscal, s->fp, time, dt0, (int)explicit_step, res_dev(s, s->slot), 0, s->ny,

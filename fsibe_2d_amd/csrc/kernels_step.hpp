@@ -64,10 +64,8 @@ __device__ __forceinline__ double2 live(const double2 *__restrict__ row, int k, 
   return k < kc ? v : make_double2(0.0, 0.0);
 }
 
-// fn(cut) for rows of H entries stored up to kc: decided once a row, since the
-// selects cost a whole row some percent of its kernel's time (K2 of the first
-// step of a call, 1024 rows of 512: 18.3 us with them, 17.1 without; 4096 rows
-// 54.5 and 52.3)
+// fn(cut) for rows of H entries stored up to kc: decided once a row instead of at
+// each load
 template <class Fn>
 __device__ __forceinline__ void with_cut(int H, int kc, const Fn &fn) {
   if (H <= kCutH || kc >= H) fn(std::false_type{});
@@ -388,7 +386,7 @@ __device__ void step_scalars(const double *__restrict__ umax_part, int nparts, D
 // K2: nonlinear term, penalisation and sponge in physical space (one row/WG)
 // cal_nlk, NavierStokes.f90:39-52 and :88-164
 // ============================================================================
-template <class FX>
+template <bool CUT, class FX>
 __device__ __forceinline__ void rows_nl_body(const double2 *__restrict__ A, const double2 *__restrict__ B,
                                                     const double *__restrict__ u1, const double *__restrict__ u2,
                                                     const double *__restrict__ ms, MaskBox mb, int penal_on,
@@ -406,15 +404,12 @@ __device__ __forceinline__ void rows_nl_body(const double2 *__restrict__ A, cons
   const bool prow = penal_on && mb.x1 >= mb.x0 && y >= mb.y0 && y <= mb.y1;
   double ps1 = 0.0, ps2 = 0.0;  // the row's sums of the penalisation term (rowpen)
   // rows: w, dw/dy, dw/dx = i kx w
-  with_cut(H, c.kc, [&](auto cut) {
-    constexpr bool CUT = decltype(cut)::value;
-    stage_rows_c2r<3>(lds, 3, H, PL, twx, tid, nt, [&](int f, int k) -> double2 {
-      if (f == 1) return live<CUT>(B + (size_t)y * H, k, H, c.kc);
-      const double2 a = live<CUT>(A + (size_t)y * H, k, H, c.kc);
-      if (f == 0) return a;
-      const double kf = (double)k * c.sx;
-      return make_double2(-kf * a.y, kf * a.x);
-    });
+  stage_rows_c2r<3>(lds, 3, H, PL, twx, tid, nt, [&](int f, int k) -> double2 {
+    if (f == 1) return live<CUT>(B + (size_t)y * H, k, H, c.kc);
+    const double2 a = live<CUT>(A + (size_t)y * H, k, H, c.kc);
+    if (f == 0) return a;
+    const double kf = (double)k * c.sx;
+    return make_double2(-kf * a.y, kf * a.x);
   });
   F.template fft<true, 3>(lds, twx, tid, nt);
   for (int n = tid; n < H; n += nt) {
@@ -1041,7 +1036,10 @@ __global__ void __launch_bounds__(FY::LB) k_cols_inv_fields(const double2 *__res
   cols_inv_fields_body(W, o0, o1, o2, o3, fsel0, fsel1, fsel2, fsel3, nfield, F, twy, c, r0_3, r1_3, blockIdx.x,
                        gridDim.x);
 }
-template <class FX>
+// CUT: columns of A, B beyond c.kc are left out.  The host chooses the instance;
+// both forms behind a branch cost rows that are cut (512 rows of 384: 14.1 us,
+// 13.5 alone).
+template <class FX, bool CUT>
 __global__ void __launch_bounds__(FX::LB) k_rows_nl(const double2 *__restrict__ A, const double2 *__restrict__ B,
                                                     const double *__restrict__ u1, const double *__restrict__ u2,
                                                     const double *__restrict__ ms, MaskBox mb, int penal_on,
@@ -1054,7 +1052,7 @@ __global__ void __launch_bounds__(FX::LB) k_rows_nl(const double2 *__restrict__ 
                                                     int rpx_zero) {
   // rows ra .. ra+na-1, then rb onwards (two row ranges; one when rb is unused)
   const int b = blockIdx.x;
-  rows_nl_body(A, B, u1, u2, ms, mb, penal_on, Rc, Rpx, F, twx, c, umax_part, nparts, sc, fl, time, dt0,
+  rows_nl_body<CUT>(A, B, u1, u2, ms, mb, penal_on, Rc, Rpx, F, twx, c, umax_part, nparts, sc, fl, time, dt0,
                explicit_step, res, b < na ? ra + b : rb + (b - na), scal && b == 0, rowpen, rpx_zero);
 }
 
@@ -1235,7 +1233,7 @@ __global__ void __launch_bounds__(FX::LB) kb_rows_nl(const RowsNlArgs *__restric
                                                      const double2 *__restrict__ twx) {
   const RowsNlArgs &a = arr[blockIdx.y];
   if ((int)blockIdx.x >= a.nblk) return;
-  rows_nl_body(a.A, a.B, a.u1, a.u2, a.ms, a.mb, a.penal_on, a.Rc, a.Rpx, F, twx, a.c, a.umax_part, a.nparts, a.sc,
+  rows_nl_body<false>(a.A, a.B, a.u1, a.u2, a.ms, a.mb, a.penal_on, a.Rc, a.Rpx, F, twx, a.c, a.umax_part, a.nparts, a.sc,
                a.fl, a.time, a.dt0, a.explicit_step, a.res, (int)blockIdx.x, blockIdx.x == 0, nullptr, a.rpx_zero);
 }
 template <class FY>
