@@ -1720,14 +1720,12 @@ extern "C" int fsibe_sim_create(const fsibe_params *pp, fsibe_sim **out) {
   {
     // every field of the grid in one allocation (22 of them: each call of
     // the allocator costs more than the fields' clearing), the ones that
-    // are read before they are written cleared.  Large fields at a distance
+    // are read before they are written cleared.  Fields at a distance
     // of exactly a power of two meet in the same memory channels: 4 KiB and 256 B
     // more between them took a step with a body at 4096^2 from 1930 to 1826 us, at
     // 1024 x 4096 from 416 to 409 (without a body 243 to 225), at 2048^2 from 325
-    // to 317, at 1024^2 from 98.5 to 96.6.  Fields below 4 MiB, which
-    // the caches hold, gain nothing (512^2 30.7 and 30.6 us) and stay together
-    const size_t len = sizeof(double2) * NH;
-    const size_t fld = ((len + 255) & ~(size_t)255) + (len >= (size_t)4 << 20 ? 4096 + 256 : 0);
+    // to 317, at 1024^2 from 98.5 to 96.6, a gradient at 512^2 from 23.8 to 23.6 ms
+    const size_t fld = ((sizeof(double2) * NH + 255) & ~(size_t)255) + 4096 + 256;
     SIMCHK(hipMalloc(&s->fields, 22 * fld));
     SIMCHK(hipMemset(s->fields, 0, 14 * fld));
     char *q = s->fields;
