@@ -43,7 +43,7 @@ KERNELS = ["create_mask", "startup_velocity", "cols_vortk_n0", "rows_nonlinear",
 
 
 def alg_bytes(name: str, nx: int, ny: int, visc: bool, box_rows: int, box_cols: int,
-              mask_px: int = 0) -> float:
+              mask_px: int = 0, mask_rows: int = 0) -> float:
     """Compulsory HBM bytes of one launch: every operand read once and every
     result written once (S = one nx*ny FP64 field = 8 nx ny bytes; a
     half-spectrum field of ny x nx/2 complex values is also S)."""
@@ -51,13 +51,16 @@ def alg_bytes(name: str, nx: int, ny: int, visc: bool, box_rows: int, box_cols: 
     rowS = 8.0 * nx
     return {
         "create_mask": 3 * 8.0 * mask_px,           # mask, mask_vx, mask_vy on the mask box
+        # as the profiled pass launches them, with nothing formed ahead: both
+        # columns and every row (the coupled loop's own K1 forms one column, 2 S)
         "cols_vortk_n0": 3 * S,                     # W0 -> A, B
-        "rows_nonlinear": 7 * S,                    # A, B, u1, u2, chi_s -> Rc, Rpx
-        # the fused column stage: Rc, Rpx (box rows), W0 and nlk(n1) inside the
+        "rows_nonlinear": 6 * S + mask_rows * rowS,  # A, B, u1, u2, chi_s -> Rc, Rpx (mask rows)
+        # the fused column stage: Rc, Rpx (mask rows), W0 and nlk(n1) inside the
         # dealiasing ellipse (pi/9 of the modes) -> nlk(n0), W1, and on the
         # two thirds of the columns that reach it omega, psi, i ky psi
         # (, -ky^2 psi on the box rows)
-        "cols_ab2_update": (1 + 2 * math.pi / 9 + 2 + 2) * S + box_rows * rowS * (1 + (2 / 3 if visc else 0)),
+        "cols_ab2_update": (1 + 2 * math.pi / 9 + 2 + 2) * S + mask_rows * rowS
+                           + (2 / 3 * box_rows * rowS if visc else 0),
         "cols_vortk_n1": (5 if visc else 4) * S,    # launched only where no fused column stage exists
         # 3 inputs (two thirds of their columns) + vor_mean r/w -> u1, u2, Rq, Rqy
         "rows_velocity_pressure": 8 * S,
@@ -633,11 +636,12 @@ def main(argv=None) -> int:
         fb = sim.box("press")[1]
         mb = sim.box("mask")[1]
         box_rows, box_cols = fb[3] - fb[2] + 1, fb[1] - fb[0] + 1
-        mask_px = max(0, mb[1] - mb[0] + 1) * max(0, mb[3] - mb[2] + 1)
+        mask_rows = max(0, mb[3] - mb[2] + 1)
+        mask_px = max(0, mb[1] - mb[0] + 1) * mask_rows
         for i, name in enumerate(KERNELS):
             if cnt[i]:
                 avg_us = 1e3 * ms[i] / cnt[i]
-                b = alg_bytes(name, n, n, True, box_rows, box_cols, mask_px)
+                b = alg_bytes(name, n, n, True, box_rows, box_cols, mask_px, mask_rows)
                 prof[name] = {"avg_us": round(avg_us, 3), "launches": int(cnt[i]),
                               "alg_bytes": b, "GBps": round(b / (avg_us * 1e-6) / 1e9, 1) if b else None}
         # dominant kernel: largest total time among the HBM-streaming kernels;
